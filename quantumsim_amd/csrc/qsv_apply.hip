@@ -17,6 +17,7 @@
 #include "qsv_common.h"
 #include "qsv_geom.h"
 #include "qsv_fused.h"
+#include "qsv_table.h"
 
 #include <algorithm>
 #include <stdlib.h>
@@ -56,19 +57,6 @@ struct PtrOp {
   __device__ __forceinline__ int64_t oout(int o) const { return off_out[o]; }
 };
 
-// Offsets and PTM in device memory (any size).  Table layout, built by the
-// host: int64 off_in[din_pad]; int64 off_out[dout_pad]; and either the PTM
-// zero padded to dout_pad x din_pad right after (padded = 1) or a separate
-// caller-owned dout x din PTM (padded = 0).
-template <typename T>
-struct TableOp {
-  const int64_t* __restrict__ off_in;
-  const int64_t* __restrict__ off_out;
-  const T* __restrict__ ptm;
-  int32_t ld;
-  int32_t padded;
-};
-
 // ---------------------------------------------------------------- small
 // din, dout <= CH: all D_in operands live in registers, outputs stream out.
 template <typename T, int CH, int VEC, bool NT, bool FULL, class Op>
@@ -106,118 +94,7 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// ---------------------------------------------------------------- table
-// Any din/dout: operands CH at a time, outputs CH at a time.
-template <typename T, int CH, int VEC>
-__global__ void __launch_bounds__(kBlock)
-    k_apply_table(const T* __restrict__ in, T* __restrict__ out, const Geom g,
-                  const TableOp<T> op) {
-  typedef typename VT<T, VEC>::t V;
-  const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= g.n_threads) return;
-  int64_t bin, bout;
-  orbit_base(g, t * VEC, bin, bout);
-
-  for (int oc = 0; oc < g.dout; oc += CH) {
-    V acc[CH];
-#pragma unroll
-    for (int o = 0; o < CH; ++o) acc[o] = V(0);
-    for (int ic = 0; ic < g.din; ic += CH) {
-      V v[CH];
-#pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        if (ic + i < g.din)
-          v[i] = *reinterpret_cast<const V*>(in + bin + op.off_in[ic + i]);
-        else
-          v[i] = V(0);
-      }
-#pragma unroll
-      for (int o = 0; o < CH; ++o) {
-        if (oc + o < g.dout) {
-          const T* prow = op.ptm + int64_t(oc + o) * op.ld + ic;
-#pragma unroll
-          for (int i = 0; i < CH; ++i) {
-            if (op.padded || ic + i < g.din) acc[o] += prow[i] * v[i];
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int o = 0; o < CH; ++o) {
-      if (oc + o < g.dout) *reinterpret_cast<V*>(out + bout + op.off_out[oc + o]) = acc[o];
-    }
-  }
-}
-
-// ------------------------------------------------------- table, batched
-// The table kernel for PTMs in device memory of any size (qutrit pairs 81 x
-// 81, qubit-qutrit 36 x 36, ...), batched (grid.y = state, each state's PTM
-// pstride elements apart, 0 = shared), with the entry offsets decoded by
-// every block into LDS from the targets' dims and strides: no host table,
-// no copy, so it is safe under graph capture.
-struct TableGeo {
-  int32_t k;
-  int32_t din_t[QSV_MAX_TARGETS], dout_t[QSV_MAX_TARGETS];
-  int64_t sin_t[QSV_MAX_TARGETS], sout_t[QSV_MAX_TARGETS];
-};
-constexpr int kTableMaxD = 1024;  // entries per side the LDS offsets hold
-
-// Offset of PTM index e on one side: mixed radix over the targets in PTM
-// axis order, the last target fastest.
-__host__ __device__ inline int64_t table_offset(int k, const int32_t* d, const int64_t* st,
-                                                int e) {
-  int64_t off = 0;
-  for (int j = k - 1; j >= 0; --j) {
-    off += int64_t(e % d[j]) * st[j];
-    e /= d[j];
-  }
-  return off;
-}
-
-template <typename T, int CH, int VEC>
-__global__ void __launch_bounds__(kBlock)
-    k_apply_table_b(const T* __restrict__ in, T* __restrict__ out, const Geom g,
-                    const TableGeo tg, const T* __restrict__ ptm, const int64_t pstride) {
-  typedef typename VT<T, VEC>::t V;
-  __shared__ int64_t so_in[kTableMaxD], so_out[kTableMaxD];
-  for (int e = threadIdx.x; e < g.din; e += kBlock)
-    so_in[e] = table_offset(tg.k, tg.din_t, tg.sin_t, e);
-  for (int e = threadIdx.x; e < g.dout; e += kBlock)
-    so_out[e] = table_offset(tg.k, tg.dout_t, tg.sout_t, e);
-  __syncthreads();
-  const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= g.n_threads) return;
-  const uint32_t b = blockIdx.y;
-  in += int64_t(b) * g.bs_in;
-  out += int64_t(b) * g.bs_out;
-  ptm += int64_t(b) * pstride;
-  int64_t bin, bout;
-  orbit_base(g, t * VEC, bin, bout);
-  for (int oc = 0; oc < g.dout; oc += CH) {
-    V acc[CH];
-#pragma unroll
-    for (int o = 0; o < CH; ++o) acc[o] = V(0);
-    for (int ic = 0; ic < g.din; ic += CH) {
-      V v[CH];
-#pragma unroll
-      for (int i = 0; i < CH; ++i)
-        v[i] = ic + i < g.din ? *reinterpret_cast<const V*>(in + bin + so_in[ic + i]) : V(0);
-#pragma unroll
-      for (int o = 0; o < CH; ++o) {
-        if (oc + o < g.dout) {
-          const T* prow = ptm + int64_t(oc + o) * g.din + ic;
-#pragma unroll
-          for (int i = 0; i < CH; ++i)
-            if (ic + i < g.din) acc[o] += prow[i] * v[i];
-        }
-      }
-    }
-#pragma unroll
-    for (int o = 0; o < CH; ++o)
-      if (oc + o < g.dout) *reinterpret_cast<V*>(out + bout + so_out[oc + o]) = acc[o];
-  }
-}
-
+constexpr int kTableMaxD = 1024;  // entries per side of the device-PTM and batched paths
 
 // ------------------------------------------------------------ LDS tiled
 // For targets near the innermost axis the orbit entries of neighbouring
@@ -939,28 +816,6 @@ static int run_ptr(const Plan& p, const void* ptm_dev, const void* in, void* out
   return dispatch_vec_small<T, CH, PtrOp>(p, op, in, out, s);
 }
 
-template <typename T, int CH, int VEC>
-static int launch_table(const Plan& p, const TableOp<T>& op, const void* in, void* out,
-                        hipStream_t s) {
-  if (p.g.n_threads == 0) return QSV_OK;
-  const dim3 grid(ceil_div_u32(p.g.n_threads, kBlock));
-  hipLaunchKernelGGL((k_apply_table<T, CH, VEC>), grid, dim3(kBlock), 0, s,
-                     static_cast<const T*>(in), static_cast<T*>(out), p.g, op);
-  QSV_CHECK_HIP(hipGetLastError());
-  return QSV_OK;
-}
-
-template <typename T>
-static int run_table(const Plan& p, const TableOp<T>& op, const void* in, void* out,
-                     hipStream_t s) {
-  if constexpr (std::is_same<T, double>::value) {
-    if (p.vec == 2) return launch_table<T, 16, 2>(p, op, in, out, s);
-  } else {
-    if (p.vec == 4) return launch_table<T, 16, 4>(p, op, in, out, s);
-  }
-  return launch_table<T, 16, 1>(p, op, in, out, s);
-}
-
 static inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 
 static bool fits_inline(int64_t din, int64_t dout) {
@@ -1050,34 +905,8 @@ static int run_fused(const Plan& p, const FusedPlan& fp, const double* ptm_f64, 
   return launch_fused(sizeof(T) == 8 ? QSV_F64 : QSV_F32, fp, p.g, p.nt, in, out, workspace, s);
 }
 
-template <typename T>
-static int run_host_table(const Plan& p, const double* ptm_f64, void* workspace,
-                          const void* in, void* out, hipStream_t s) {
-  const int64_t need = table_bytes(sizeof(T) == 8 ? QSV_F64 : QSV_F32, p.din, p.dout, true);
-  const int64_t dinp = round_up(p.din, 16), doutp = round_up(p.dout, 16);
-  std::vector<unsigned char> host(need, 0);
-  int64_t* oin = reinterpret_cast<int64_t*>(host.data());
-  int64_t* oout = oin + dinp;
-  for (int i = 0; i < p.din; ++i) oin[i] = p.off_in[i];
-  for (int o = 0; o < p.dout; ++o) oout[o] = p.off_out[o];
-  T* P = reinterpret_cast<T*>(host.data() + (dinp + doutp) * 8);
-  for (int o = 0; o < p.dout; ++o)
-    for (int i = 0; i < p.din; ++i) P[o * dinp + i] = T(ptm_f64[int64_t(o) * p.din + i]);
-  // pageable source: the runtime copies it to staging before returning
-  QSV_CHECK_HIP(hipMemcpyAsync(workspace, host.data(), need, hipMemcpyHostToDevice, s));
-  const unsigned char* wb = static_cast<const unsigned char*>(workspace);
-  TableOp<T> op{reinterpret_cast<const int64_t*>(wb),
-                reinterpret_cast<const int64_t*>(wb) + dinp,
-                reinterpret_cast<const T*>(wb + (dinp + doutp) * 8), int32_t(dinp), 1};
-  return run_table<T>(p, op, in, out, s);
-}
-
-
 // TableGeo of a plan, checked against the plan's own offsets.
 static int make_table_geo(const Plan& p, TableGeo& tg) {
-  QSV_CHECK_ARG(p.din <= kTableMaxD && p.dout <= kTableMaxD,
-                "PTM of %d x %d: the table kernel takes up to %d entries per side", p.dout,
-                p.din, kTableMaxD);
   memset(&tg, 0, sizeof(tg));
   tg.k = p.k;
   for (int j = 0; j < p.k; ++j) {
@@ -1096,25 +925,34 @@ static int make_table_geo(const Plan& p, TableGeo& tg) {
   return QSV_OK;
 }
 
+// Host PTM of any size: copied to the workspace in the state's type, then
+// applied as a device PTM.
 template <typename T>
-static int run_table_b(const Plan& p, const void* ptm_dev, int64_t pstride, uint32_t batch,
-                       const void* in, void* out, hipStream_t s) {
+static int run_host_table(const Plan& p, const double* ptm_f64, void* workspace,
+                          const void* in, void* out, hipStream_t s) {
   TableGeo tg;
   const int rc = make_table_geo(p, tg);
   if (rc) return rc;
-  if (p.g.n_threads == 0 || batch == 0) return QSV_OK;
-  const dim3 grid(ceil_div_u32(p.g.n_threads, kBlock), batch);
-  const T* pt = static_cast<const T*>(ptm_dev);
-  if (p.vec == 16 / int(sizeof(T)))
-    hipLaunchKernelGGL((k_apply_table_b<T, 16, 16 / sizeof(T)>), grid, dim3(kBlock), 0, s,
-                       static_cast<const T*>(in), static_cast<T*>(out), p.g, tg, pt, pstride);
-  else
-    hipLaunchKernelGGL((k_apply_table_b<T, 16, 1>), grid, dim3(kBlock), 0, s,
-                       static_cast<const T*>(in), static_cast<T*>(out), p.g, tg, pt, pstride);
-  QSV_CHECK_HIP(hipGetLastError());
-  return QSV_OK;
+  std::vector<T> host(size_t(p.dout) * p.din);
+  for (size_t e = 0; e < host.size(); ++e) host[e] = T(ptm_f64[e]);
+  // pageable source: the runtime copies it to staging before returning
+  QSV_CHECK_HIP(hipMemcpyAsync(workspace, host.data(), host.size() * sizeof(T),
+                               hipMemcpyHostToDevice, s));
+  return launch_table(sizeof(T) == 8 ? QSV_F64 : QSV_F32, p.g, p.g.n_threads * p.vec, tg, in, out,
+                      workspace, 0, 1, s);
 }
 
+// Device PTMs of any size, one per state (pstride 0: one for all).
+static int run_table_b(int dtype, const Plan& p, const void* ptm_dev, int64_t pstride,
+                       uint32_t batch, const void* in, void* out, hipStream_t s) {
+  QSV_CHECK_ARG(p.din <= kTableMaxD && p.dout <= kTableMaxD,
+                "PTM of %d x %d: the table kernel takes up to %d entries per side", p.dout,
+                p.din, kTableMaxD);
+  TableGeo tg;
+  const int rc = make_table_geo(p, tg);
+  if (rc) return rc;
+  return launch_table(dtype, p.g, p.g.n_threads * p.vec, tg, in, out, ptm_dev, pstride, batch, s);
+}
 
 }  // namespace qsv
 
@@ -1211,8 +1049,7 @@ extern "C" int qsv_apply_ptm_dev_strided(int dtype, const void* in, void* out, i
   // (no host table, no copy)
   (void)workspace;
   (void)workspace_bytes;
-  return dtype == QSV_F64 ? run_table_b<double>(p, ptm_dev, 0, 1, in, out, s)
-                          : run_table_b<float>(p, ptm_dev, 0, 1, in, out, s);
+  return run_table_b(dtype, p, ptm_dev, 0, 1, in, out, s);
 }
 
 extern "C" int qsv_apply_ptm_dev(int dtype, const void* in, void* out, int rank,
@@ -1340,6 +1177,79 @@ static int emulate_lds(const Plan& p, const LdsPlan& lp, int elem_bytes, const d
       }
   }
   return check_coverage(p, written, "lds");
+}
+
+// Replays k_apply_table wave by wave: the staged PTM in fragment order, the
+// entry loads (past-the-end columns and orbits included), the MFMA
+// contraction in hardware index order and the accumulator stores.
+static int emulate_table(const Plan& p, int elem_bytes, const double* ptm, const double* in,
+                         double* out) {
+  TableGeo tg;
+  const int rc = make_table_geo(p, tg);
+  if (rc) return rc;
+  const uint32_t n_orbits = p.g.n_threads * p.vec;
+  const int MB = table_row_blocks(p.dout), NB = elem_bytes == 4 ? 2 : 1, rows = 16 * MB;
+  QSV_CHECK_ARG(MB >= 1 && MB <= kTableMaxRowBlocks, "table: %d row blocks", MB);
+  const uint32_t cols = 16 * NB, tiles = (n_orbits + cols - 1) / cols;
+  std::vector<int> written(p.n_out, 0);
+  for (int row0 = 0; row0 < p.dout; row0 += rows)
+    for (uint32_t t = 0; t < tiles; ++t)
+      for (int nb = 0; nb < NB; ++nb) {
+        std::vector<double> acc(size_t(64) * MB * 4, 0.0);
+        int64_t bin[16], bout[16];
+        uint32_t m[16];
+        for (int n = 0; n < 16; ++n) {
+          m[n] = t * cols + 16 * nb + n;
+          orbit_base(p.g, m[n] < n_orbits ? m[n] : n_orbits - 1, bin[n], bout[n]);
+        }
+        for (int c0 = 0; c0 < p.din; c0 += kTableCols) {
+          std::vector<double> As(size_t(kTableCols) / 4 * MB * 64, 0.0);
+          std::vector<int> staged(As.size(), 0);
+          for (int r = 0; r < rows; ++r)
+            for (int kk = 0; kk < kTableCols; ++kk) {
+              const int slot = table_slot(MB, r, kk);
+              QSV_CHECK_ARG(slot >= 0 && slot < int(As.size()) && staged[slot]++ == 0,
+                            "table: PTM slot %d", slot);
+              if (row0 + r < p.dout && c0 + kk < p.din)
+                As[slot] = ptm[int64_t(row0 + r) * p.din + c0 + kk];
+            }
+          const int kn = std::min(kTableCols, p.din - c0);
+          for (int s = 0; 4 * s < kn; ++s) {
+            double B[64];
+            for (int lane = 0; lane < 64; ++lane) {
+              const int n = lane & 15, k = 4 * s + (lane >> 4);
+              const int64_t a =
+                  bin[n] + table_offset(tg.k, tg.din_t, tg.sin_t, c0 + (k < kn ? k : 0));
+              QSV_CHECK_ARG(a >= 0 && a < p.n_in, "table: load %lld out of bounds", (long long)a);
+              B[lane] = k < kn ? in[a] : 0.0;
+            }
+            for (int lane = 0; lane < 64; ++lane)
+              for (int mb = 0; mb < MB; ++mb)
+                for (int r = 0; r < 4; ++r) {
+                  const int n = lane & 15, j = lane >> 4;
+                  const int row = elem_bytes == 8 ? j + 4 * r : 4 * j + r;
+                  for (int q = 0; q < 4; ++q)
+                    acc[(size_t(lane) * MB + mb) * 4 + r] +=
+                        As[(s * MB + mb) * 64 + row + 16 * q] * B[n + 16 * q];
+                }
+          }
+        }
+        for (int lane = 0; lane < 64; ++lane) {
+          const int n = lane & 15, j = lane >> 4;
+          if (m[n] >= n_orbits) continue;
+          for (int mb = 0; mb < MB; ++mb)
+            for (int r = 0; r < 4; ++r) {
+              const int row = row0 + 16 * mb + (elem_bytes == 8 ? j + 4 * r : 4 * j + r);
+              if (row >= p.dout) continue;
+              const int64_t a = bout[n] + table_offset(tg.k, tg.dout_t, tg.sout_t, row);
+              QSV_CHECK_ARG(a >= 0 && a < p.n_out, "table: store %lld out of bounds",
+                            (long long)a);
+              out[a] = acc[(size_t(lane) * MB + mb) * 4 + r];
+              ++written[a];
+            }
+        }
+      }
+  return check_coverage(p, written, "table");
 }
 
 // Replays k_fused64 / k_fused256 lane by lane: the B-fragment loads (with
@@ -1473,7 +1383,11 @@ extern "C" int qsv_emulate_apply_ptm(int dtype, const double* in, double* out, i
     if (path_out) *path_out = 4 | (fp.vi << 4) | (fp.vo << 8) | (fp.vn << 12);
     return emulate_fused(p, es, ptm_f64, in, out);
   }
-  if (path_out) *path_out = fits_inline(p.din, p.dout) ? 1 : 3;
+  if (!fits_inline(p.din, p.dout)) {
+    if (path_out) *path_out = 3;
+    return emulate_table(p, es, ptm_f64, in, out);
+  }
+  if (path_out) *path_out = 1;
   return emulate_direct(p, ptm_f64, in, out);
 }
 
@@ -1530,9 +1444,7 @@ extern "C" int qsv_apply_ptm_batched_tiled(int dtype, const void* in, void* out,
     // kernel with the offsets decoded on the device
     QSV_CHECK_ARG(!tile || tile->kernel == QSV_KERNEL_AUTO,
                   "%d x %d PTMs take no launch shape", p.dout, p.din);
-    return dtype == QSV_F64
-               ? run_table_b<double>(p, ptm_dev, ptm_batch_stride, uint32_t(batch), in, out, s)
-               : run_table_b<float>(p, ptm_dev, ptm_batch_stride, uint32_t(batch), in, out, s);
+    return run_table_b(dtype, p, ptm_dev, ptm_batch_stride, uint32_t(batch), in, out, s);
   }
   p.batch = uint32_t(batch);
   const bool small = std::max(p.din, p.dout) <= 4;
@@ -1568,11 +1480,11 @@ extern "C" int qsv_emulate_apply_ptm_tiled(int dtype, const double* in, double* 
     // the batched table kernel: offsets as the kernel decodes them
     QSV_CHECK_ARG(!tile || tile->kernel == QSV_KERNEL_AUTO,
                   "%d x %d PTMs take no launch shape", p.dout, p.din);
-    TableGeo tg;
-    const int rt = make_table_geo(p, tg);
-    if (rt) return rt;
+    QSV_CHECK_ARG(p.din <= kTableMaxD && p.dout <= kTableMaxD,
+                  "PTM of %d x %d: the table kernel takes up to %d entries per side", p.dout,
+                  p.din, kTableMaxD);
     if (path_out) *path_out = 3;
-    return emulate_direct(p, ptm_f64, in, out);
+    return emulate_table(p, es, ptm_f64, in, out);
   }
   LdsPlan lp;
   if (make_lds_plan(p, es, lp, tile)) {
