@@ -205,6 +205,45 @@ int qsv_circuits_forward(int dtype, int n_circuits, const qsv_circuit* circs_dev
                          const qsv_gate* gates_dev, const void* ptms, void* traj,
                          double* pops, int max_qubits, void* stream);
 
+/* Qubit circuits applied several gates to a pass over one float64 vector
+ * (n_qubits axes of dimension 4, element strides `strides`, in C order).
+ * Gates: ks[g] = 1 or 2 targets at targets[2 g], targets[2 g + 1]; ptms holds
+ * their row-major 4^k x 4^k PTMs (out..., in...), one after the other.
+ *   qsv_circuit_create   composes the gates into two-qubit blocks and plans
+ *                        the passes (host memory only); *plan_out is freed
+ *                        with qsv_circuit_destroy.  QSV_ENOTSUP: strides the
+ *                        passes cannot read in aligned runs.
+ *   qsv_circuit_passes   number of passes
+ *   qsv_circuit_table    writes the blocks' tables (qsv_circuit_table_bytes)
+ *                        to host memory; the caller copies them to the device
+ *   qsv_circuit_run      launches the passes: in -> out, the later ones in
+ *                        place on out (in is only read; both may be the same)
+ * The same gates fused into dense blocks of up to max_qudits qubits (the
+ * blocks and order of quantumsim_amd.fusion.fuse):
+ *   qsv_circuit_blocks_create  plans them; freed with qsv_circuit_blocks_destroy
+ *   qsv_circuit_blocks_count   their number
+ *   qsv_circuit_block_qubits   a block's qubits, ascending; returns how many
+ *   qsv_circuit_block_ptm      its row-major 4^k x 4^k PTM */
+int qsv_circuit_create(int n_qubits, const int64_t* strides, int n_gates, const int32_t* ks,
+                       const int32_t* targets, const double* ptms,
+                       void** plan_out);
+void qsv_circuit_destroy(void* plan);
+int qsv_circuit_passes(const void* plan);
+int64_t qsv_circuit_table_bytes(const void* plan);
+int qsv_circuit_table(const void* plan, void* host);
+int qsv_circuit_run(const void* plan, const void* in, void* out, const void* table_dev,
+                    void* stream);
+int qsv_circuit_blocks_create(int n_qubits, int n_gates, const int32_t* ks,
+                              const int32_t* targets, const double* ptms, int max_qudits,
+                              void** blocks_out);
+void qsv_circuit_blocks_destroy(void* blocks);
+int qsv_circuit_blocks_count(const void* blocks);
+int qsv_circuit_block_qubits(const void* blocks, int index, int32_t* qubits);
+int qsv_circuit_block_ptm(const void* blocks, int index, double* ptm);
+/* CPU replay of the passes on v (float64, the plan's layout), every access
+ * checked. */
+int qsv_emulate_circuit(const void* plan, double* v);
+
 /* Adjoint of qsv_circuits_forward: from dL/dpops (float64) and the forward
  * trajectory, writes dL/dP of every gate (float64, fixed summation order)
  * into dptms at the gate's PTM offset.  One persistent launch. */

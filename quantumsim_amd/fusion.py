@@ -14,9 +14,14 @@ its own qudits fits ``max_qudits`` (ties: the subset holding more gates);
 the touched blocks left out are emitted first (they act on a qudit of the
 gate, so they must precede it).  At the end every open block is emitted.
 Square PTMs (same input and output dimension per qudit) only.
+
+``apply_circuit`` runs qubit circuits without forming these blocks: in passes
+over the vector that each apply several two-qubit gates from LDS.
 """
 import itertools
 import numpy as np
+
+from . import _native as nat
 
 __all__ = ['fuse', 'fuse_plan', 'FusedGate', 'embed_ptm', 'embed_ptm_batched', 'fuse_batched',
            'apply_circuit']
@@ -203,15 +208,132 @@ def fuse_batched(gates, dims, max_qudits=3, plan=None):
     return out
 
 
+class CircuitPasses:
+    """A qubit circuit planned as passes over a float64 vector (qsv_circuit_*):
+    ``ks``, ``targets`` (two per gate) and the concatenated float64 ``ptms``
+    for a vector of n qubits with element strides ``strides``."""
+
+    def __init__(self, n, strides, ks, targets, ptms):
+        import ctypes
+        self._lib = nat.lib()
+        self.handle = None
+        handle = ctypes.c_void_p()
+        nat.check(self._lib.qsv_circuit_create(
+            n, nat.i64(strides), len(ks), ks.ctypes.data_as(nat._c_i32p),
+            targets.ctypes.data_as(nat._c_i32p), ptms.ctypes.data_as(nat._c_f64p),
+            ctypes.byref(handle)), 'apply_circuit')
+        self.handle = handle.value
+
+    def __del__(self):
+        if self.handle is not None:
+            self._lib.qsv_circuit_destroy(self.handle)
+
+    @property
+    def passes(self):
+        return self._lib.qsv_circuit_passes(self.handle)
+
+    def table(self, device):
+        """The blocks' tables on ``device``, copied from pinned memory on the
+        current stream."""
+        import torch
+        n = self._lib.qsv_circuit_table_bytes(self.handle)
+        host = torch.empty(max(n, 1), dtype=torch.uint8, pin_memory=True)
+        nat.check(self._lib.qsv_circuit_table(self.handle, host.data_ptr()), 'apply_circuit')
+        return host.to(device, non_blocking=True)
+
+    def run(self, src, dst, table, stream):
+        nat.check(self._lib.qsv_circuit_run(self.handle, src, dst, table, stream),
+                  'apply_circuit')
+
+
+class QubitBlocks:
+    """``fuse`` for the circuits ``_qubit_gates`` takes, planned and composed
+    in the library: the same blocks in the same order, PTMs equal to
+    rounding.  Iterating composes one block at a time: (ptm, qubits)."""
+
+    def __init__(self, n, ks, targets, ptms, max_qudits):
+        import ctypes
+        self._lib = nat.lib()
+        self.handle = None
+        handle = ctypes.c_void_p()
+        nat.check(self._lib.qsv_circuit_blocks_create(
+            n, len(ks), ks.ctypes.data_as(nat._c_i32p), targets.ctypes.data_as(nat._c_i32p),
+            ptms.ctypes.data_as(nat._c_f64p), int(max_qudits), ctypes.byref(handle)), 'fuse')
+        self.handle = handle.value
+
+    def __del__(self):
+        if self.handle is not None:
+            self._lib.qsv_circuit_blocks_destroy(self.handle)
+
+    def __len__(self):
+        return self._lib.qsv_circuit_blocks_count(self.handle)
+
+    def __iter__(self):
+        qubits = np.zeros(32, dtype=np.int32)
+        for i in range(len(self)):
+            k = nat.check(self._lib.qsv_circuit_block_qubits(
+                self.handle, i, qubits.ctypes.data_as(nat._c_i32p)), 'fuse')
+            ptm = np.empty((4,) * (2 * k))
+            nat.check(self._lib.qsv_circuit_block_ptm(
+                self.handle, i, ptm.ctypes.data_as(nat._c_f64p)), 'fuse')
+            yield ptm, tuple(int(q) for q in qubits[:k])
+
+
+def _qubit_gates(gates, n):
+    """(ks, targets, ptms) arrays of a circuit of 1- and 2-qubit gates with
+    real square PTMs on n qubits, or None if it holds any other gate."""
+    ks, targets, ptms = [], [], []
+    for ptm, qudits in gates:
+        p = np.asarray(ptm)
+        k = len(qudits)
+        if k not in (1, 2) or p.shape != (4,) * (2 * k) or p.dtype.kind not in 'fiub':
+            return None
+        q = [int(t) for t in qudits]
+        if min(q) < 0 or max(q) >= n or (k == 2 and q[0] == q[1]):
+            return None
+        ks.append(k)
+        targets += q if k == 2 else (q[0], -1)
+        ptms.append(p.reshape(-1))
+    return (np.array(ks, dtype=np.int32), np.array(targets, dtype=np.int32),
+            np.concatenate(ptms).astype(np.float64, copy=False))
+
+
+def _native_circuit(pv, gates):
+    """_qubit_gates' arrays where the library plans the circuit: a
+    PauliVectorHIP of 2 to 16 qubits in full bases; else None."""
+    from .pauli_vectors import PauliVectorHIP
+    if not isinstance(pv, PauliVectorHIP) or type(pv).apply_ptm is not PauliVectorHIP.apply_ptm:
+        return None
+    n = pv.n_qubits
+    if not 2 <= n <= 16 or pv.data_shape != (4,) * n or pv.dim_pauli != (4,) * n:
+        return None
+    return _qubit_gates(gates, n)
+
+
 def apply_circuit(pv, gates, max_qudits=3):
     """Apply ``gates`` = [(ptm, qudits), ...] (PTMs in ``pv``'s bases) to the
     Pauli vector ``pv``, fused into blocks of up to ``max_qudits`` qudits
-    (0 or 1: gate by gate).  Returns the number of PTM applications made."""
+    (0 or 1: gate by gate).  Returns the number of blocks.
+
+    On float64 vectors, circuits of 1- and 2-qubit gates on qubits in full
+    bases run in passes that each apply several two-qubit blocks from LDS
+    (csrc/qsv_slab.hip): the same product, rounded in another order.  Float32
+    vectors keep the blocks, whose rounding the populations of a float32 run
+    carry to their last digit; so do circuits of one block (one pass either
+    way), layouts without aligned runs and graph capture (the passes' tables
+    are copied from host memory).  Any other circuit is fused by ``fuse``."""
     if max_qudits is None or max_qudits <= 1:
         for ptm, qudits in gates:
             pv.apply_ptm(np.asarray(ptm), *qudits)
         return len(gates)
-    fused = fuse(gates, list(pv.dim_pauli), max_qudits)
-    for f in fused:
-        pv.apply_ptm(f.ptm, *f.qudits)
+    gates = list(gates)
+    arrays = _native_circuit(pv, gates) if gates else None
+    if arrays is None:
+        fused = fuse(gates, list(pv.dim_pauli), max_qudits)
+    else:
+        fused = QubitBlocks(pv.n_qubits, *arrays, max_qudits)
+        if len(fused) > 1 and pv.run_passes(*arrays):
+            return len(fused)
+    for ptm, qudits in fused:
+        pv.apply_ptm(ptm, *qudits)
     return len(fused)

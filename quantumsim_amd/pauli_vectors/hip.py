@@ -334,6 +334,34 @@ class PauliVectorHIP(PauliVectorBase):
         self._used_here(self._store, out)
         self._swap_in(out, extent, new_shape, new_str)
 
+    def run_passes(self, ks, targets, ptms):
+        """Apply a circuit of 1- and 2-qubit gates (fusion.CircuitPasses'
+        arrays) in passes of several gates each; False, with nothing done,
+        on float32 vectors, under graph capture and where the layout has no
+        such passes (see fusion.apply_circuit)."""
+        from ..fusion import CircuitPasses
+        if self._dtype != torch.float64 or self._store.data_ptr() % 16 or \
+                torch.cuda.is_current_stream_capturing():
+            return False
+        try:
+            plan = CircuitPasses(len(self._shape), self._pstr, ks, targets, ptms)
+        except NotImplementedError:
+            return False
+        extent = self._data.numel()
+        out = self._take_spare(extent)
+        # the first pass writes the spare buffer, the others work in place
+        # there: the current one is only read
+        table = plan.table(self._device)
+        try:
+            plan.run(self._store.data_ptr(), out.data_ptr(), table.data_ptr(),
+                     _stream(self._device))
+        except Exception:
+            self._spare = out
+            raise
+        self._used_here(self._store, out)
+        self._swap_in(out, extent, self._shape, self._pstr)
+        return True
+
     # ------------------------------------------------------------ readouts
     def _diag_plan(self):
         key = tuple(id(b) for b in self.bases) + (self._device,)
