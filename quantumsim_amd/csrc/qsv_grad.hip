@@ -1008,7 +1008,7 @@ int launch_apply64q(const FusedPlan& fp, const Geom& g, bool nt, const void* in,
 // the entry offsets decoded by the kernel (mixed radix, last target fastest).
 constexpr int kGradBigMaxSide = 256;
 constexpr int kGradBigMaxEntries = 8192;  // dout x din
-constexpr int kGradBigOrbits = 8;         // orbits staged in LDS per step
+constexpr int kGradBigOrbits = 16;        // orbits staged in LDS per step
 constexpr int kGradBigBlocks = 64;
 struct BigGeo {
   int32_t k;
@@ -1026,86 +1026,126 @@ __host__ __device__ inline int64_t big_offset(int k, const int32_t* d, const int
 }
 
 // PTMs above 64 x 64 (qutrit pairs, ...): dP[o][i] = sum over orbits of
-// ybar[o] x[i] on the VALU in float64.  A block takes chunks of
-// kGradBigOrbits orbits (chunk c, c + gridDim.x, ...), stages their x and
-// ybar entries in LDS (offsets decoded from the targets' dims and strides),
-// and thread t accumulates entries (o, i) = t, t + kBlock, ... of the
-// block's partial tile (same layout as the other gradient kernels, summed
-// by k_ptm_grad_final).
-constexpr int kGradBigPerThread = kGradBigMaxEntries / kBlock;
+// ybar[o] x[i] on v_mfma_f64_16x16x4f64.  A block takes chunks of
+// kGradBigOrbits orbits (chunk c, c + gridDim.x, ...) and stages their x and
+// ybar entries in LDS (offsets decoded from the targets' dims and strides;
+// float32 states widened); the 16 x 16 tiles of the output go round the four
+// waves, at most kGradBigTiles each (256 x 32 or 241 x 33: 48 tiles; 81 x 81:
+// 36), a tile taking four k-steps of four orbits a chunk.  Same partial layout
+// as the other gradient kernels, summed by k_ptm_grad_final.
+//
+// Bound: 81 x 81 is 40 flop per byte of x and ybar, so the matrix cores (26
+// padded to 96 x 96 flop per flop asked: 1.4).  Measured on 8 states of six
+// qutrits (34 MB each of x and ybar): the float64 VALU kernel this replaced,
+// with each thread reading two LDS words per multiply-add, 229 us, this one
+// 69 us.
+//
+// along_entries: staging threads walk the entries of an orbit (the innermost
+// axis is a target), else the orbits of an entry.
+constexpr int kGradBigTiles = 12;
+
+// LDS row of d entries: an odd multiple of 16 doubles, so that two of the four
+// rows an operand read touches fall on the other half of the banks.
+__host__ __device__ inline int grad_big_row(int d) { return ((d + 15) & ~15) | 16; }
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     k_ptm_grad_big(const T* __restrict__ x, const T* __restrict__ ybar, const Geom g,
-                   const BigGeo bg, const uint32_t n_orbits, double* __restrict__ partial) {
+                   const BigGeo bg, const uint32_t n_orbits, const int along_entries,
+                   double* __restrict__ partial) {
+  typedef typename Mfma<double>::acc Acc;
   __shared__ int64_t so_in[kGradBigMaxSide], so_out[kGradBigMaxSide];
-  __shared__ double sx[kGradBigOrbits * kGradBigMaxSide], sy[kGradBigOrbits * kGradBigMaxSide];
+  __shared__ int64_t base_in[kGradBigOrbits], base_out[kGradBigOrbits];
+  __shared__ double sm[kGradBigOrbits * 320];
   const uint32_t b = blockIdx.y;
   x += int64_t(b) * g.bs_in;
   ybar += int64_t(b) * g.bs_out;
   const int tid = threadIdx.x, din = g.din, dout = g.dout, dd = din * dout;
+  const int lane = tid & 63, w = tid >> 6, n = lane & 15, kk = lane >> 4;
+  const int rx = grad_big_row(din), ry = grad_big_row(dout);
+  double* sx = sm;
+  double* sy = sm + kGradBigOrbits * rx;
   for (int e = tid; e < din; e += kBlock) so_in[e] = big_offset(bg.k, bg.din_t, bg.sin_t, e);
   for (int e = tid; e < dout; e += kBlock) so_out[e] = big_offset(bg.k, bg.dout_t, bg.sout_t, e);
-  double acc[kGradBigPerThread];
+  const int ct = (din + 15) / 16, tiles = ct * ((dout + 15) / 16);
+  Acc acc[kGradBigTiles];
 #pragma unroll
-  for (int r = 0; r < kGradBigPerThread; ++r) acc[r] = 0.0;
+  for (int r = 0; r < kGradBigTiles; ++r) acc[r] = Acc(0);
+  auto stage = [&](const T* src, const int64_t* base, const int64_t* off, int d, int row,
+                   uint32_t m0, double* dst) {
+    for (int f = tid; f < kGradBigOrbits * d; f += kBlock) {
+      const int ol = along_entries ? f / d : f & (kGradBigOrbits - 1);
+      const int e = along_entries ? f - ol * d : f / kGradBigOrbits;
+      // orbits past the last: zeros, which add nothing
+      dst[ol * row + e] = m0 + ol < n_orbits ? double(src[base[ol] + off[e]]) : 0.0;
+    }
+  };
   const uint32_t nchunks = (n_orbits + kGradBigOrbits - 1) / kGradBigOrbits;
-  __syncthreads();
   for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-    for (int f = tid; f < kGradBigOrbits * din; f += kBlock) {
-      const int ol = f / din, i = f - ol * din;
-      const uint32_t m = c * kGradBigOrbits + ol;
-      double v = 0.0;
-      if (m < n_orbits) {
-        int64_t bin, bout;
-        orbit_base(g, m, bin, bout);
-        v = double(x[bin + so_in[i]]);
-      }
-      sx[ol * kGradBigMaxSide + i] = v;
-    }
-    for (int f = tid; f < kGradBigOrbits * dout; f += kBlock) {
-      const int ol = f / dout, o = f - ol * dout;
-      const uint32_t m = c * kGradBigOrbits + ol;
-      double v = 0.0;
-      if (m < n_orbits) {
-        int64_t bin, bout;
-        orbit_base(g, m, bin, bout);
-        v = double(ybar[bout + so_out[o]]);
-      }
-      sy[ol * kGradBigMaxSide + o] = v;
+    const uint32_t m0 = c * kGradBigOrbits;
+    if (tid < kGradBigOrbits) {
+      int64_t bi, bo;
+      orbit_base(g, m0 + tid < n_orbits ? m0 + tid : n_orbits - 1, bi, bo);
+      base_in[tid] = bi;
+      base_out[tid] = bo;
     }
     __syncthreads();
+    stage(x, base_in, so_in, din, rx, m0, sx);
+    stage(ybar, base_out, so_out, dout, ry, m0, sy);
+    __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kGradBigPerThread; ++r) {
-      const int j = tid + r * kBlock;
-      if (j < dd) {
-        const int o = j / din, i = j - o * din;
-        double s = acc[r];
+    for (int r = 0; r < kGradBigTiles; ++r) {
+      const int t = w + 4 * r;
+      if (t < tiles) {
+        const double* pa = sy + kk * ry + 16 * (t / ct) + n;
+        const double* pb = sx + kk * rx + 16 * (t % ct) + n;
 #pragma unroll
-        for (int ol = 0; ol < kGradBigOrbits; ++ol)
-          s += sy[ol * kGradBigMaxSide + o] * sx[ol * kGradBigMaxSide + i];
-        acc[r] = s;
+        for (int s = 0; s < kGradBigOrbits / 4; ++s)
+          acc[r] = Mfma<double>::op(pa[4 * s * ry], pb[4 * s * rx], acc[r]);
       }
     }
-    __syncthreads();
   }
   double* out = partial + (int64_t(b) * gridDim.x + blockIdx.x) * dd;
 #pragma unroll
-  for (int r = 0; r < kGradBigPerThread; ++r) {
-    const int j = tid + r * kBlock;
-    if (j < dd) out[j] = acc[r];
+  for (int r = 0; r < kGradBigTiles; ++r) {
+    const int t = w + 4 * r;
+    if (t >= tiles) continue;
+    const int i = 16 * (t % ct) + n;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int o = 16 * (t / ct) + kk + 4 * q;
+      if (o < dout && i < din) out[o * din + i] = acc[r][q];
+    }
   }
 }
 
+// One thread per (b, o, i): the block partials summed in order.  Sixteen loads
+// are in flight at a time: one after the other, a thread's 64 partials took
+// 13 us (their latencies) on a few blocks of the chip; 4.2 us now.
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     k_ptm_grad_final(const double* __restrict__ partial, int nblocks, int dd,
                      T* __restrict__ out, double scale_out_accumulate) {
-  // one thread per (b, o, i): fixed-order sum over the block partials
+  constexpr int U = 16;
   const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   const int64_t b = blockIdx.y;
   if (j >= dd) return;
+  const double* p = partial + b * nblocks * dd + j;
   double s = 0.0;
-  for (int k = 0; k < nblocks; ++k) s += partial[(b * nblocks + k) * dd + j];
+  int k = 0;
+  for (; k + U <= nblocks; k += U) {
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = p[int64_t(k + u) * dd];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += v[u];
+  }
+  double v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = k + u < nblocks ? p[int64_t(k + u) * dd] : 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (k + u < nblocks) s += v[u];
   if (scale_out_accumulate != 0.0)
     out[b * dd + j] = T(double(out[b * dd + j]) + s);
   else
@@ -1123,6 +1163,16 @@ struct GradPlan {
   int big;   // above 64 on a side: k_ptm_grad_big, offsets decoded on the device
   BigGeo bg;
 };
+
+// k_ptm_grad_big: the innermost axis is a target on both sides.
+static int grad_big_along(const GradPlan& p) {
+  bool in = false, out = false;
+  for (int j = 0; j < p.bg.k; ++j) {
+    in = in || (p.bg.sin_t[j] == 1 && p.bg.din_t[j] > 1);
+    out = out || (p.bg.sout_t[j] == 1 && p.bg.dout_t[j] > 1);
+  }
+  return in && out;
+}
 
 // Tile of the LDS-staged gradient (float64 states only).
 constexpr int kGrad64sTile = 16;
@@ -1297,11 +1347,12 @@ static int grad64_blocks(uint32_t n_orbits, int batch) {
   return int(b < 1 ? 1 : (b > kGrad64Blocks ? kGrad64Blocks : b));
 }
 
-// Above 64 x 64: at least 256 orbits per block, ~1024 blocks over the
-// batch, at most kGradBigBlocks per state (partial tiles up to 64 KB).
+// Above 64 x 64: at least 64 orbits per block (four chunks), ~512 blocks over
+// the batch (two per CU), at most kGradBigBlocks per state (partial tiles up to
+// 64 KB).
 static int grad_big_blocks(uint32_t n_orbits, int batch) {
-  uint32_t b = (n_orbits + 255) / 256;
-  const uint32_t fill = uint32_t((1024 + std::max(batch, 1) - 1) / std::max(batch, 1));
+  uint32_t b = (n_orbits + 63) / 64;
+  const uint32_t fill = uint32_t((512 + std::max(batch, 1) - 1) / std::max(batch, 1));
   b = std::min(b, fill);
   return int(b < 1 ? 1 : (b > kGradBigBlocks ? kGradBigBlocks : b));
 }
@@ -1523,7 +1574,7 @@ static void launch_grad(const GradPlan& p, int vn, bool quad, dim3 grid, const v
   const T* yy = static_cast<const T*>(ybar);
   if (p.big) {
     hipLaunchKernelGGL(k_ptm_grad_big<T>, grid, dim3(kBlock), 0, s, xx, yy, p.g, p.bg,
-                       p.n_orbits, partial);
+                       p.n_orbits, grad_big_along(p), partial);
     return;
   }
   if (grad_wide(p)) {
@@ -2077,56 +2128,62 @@ static int emulate_grad64s(const GradPlan& p, int es, const double* x, const dou
 
 // Host replay of k_ptm_grad_big + k_ptm_grad_final for one state: the
 // decoded offsets, every staged load in bounds, every (entry, orbit) staged
-// exactly once, the LDS slots inside their rows.
+// exactly once, the LDS slots inside the array, the MFMA tiles lane by lane.
 static int emulate_grad_big(const GradPlan& p, const double* x, const double* ybar, int nb,
                             double* dptm) {
   const int din = p.din, dout = p.dout, dd = din * dout;
-  std::vector<int64_t> oin(din), oout(dout);
-  for (int e = 0; e < din; ++e) oin[e] = big_offset(p.bg.k, p.bg.din_t, p.bg.sin_t, e);
-  for (int e = 0; e < dout; ++e) oout[e] = big_offset(p.bg.k, p.bg.dout_t, p.bg.sout_t, e);
-  const uint32_t nchunks = (p.n_orbits + kGradBigOrbits - 1) / kGradBigOrbits;
+  const int rx = grad_big_row(din), ry = grad_big_row(dout), along = grad_big_along(p);
+  const int ct = (din + 15) / 16, tiles = ct * ((dout + 15) / 16);
+  constexpr int NO = kGradBigOrbits, kLds = kGradBigOrbits * 320;
+  QSV_CHECK_ARG(NO * (rx + ry) <= kLds, "big gradient: %d + %d entries of LDS rows", rx, ry);
+  QSV_CHECK_ARG(tiles <= 4 * kGradBigTiles, "big gradient: %d tiles", tiles);
+  const uint32_t nchunks = (p.n_orbits + NO - 1) / NO;
   std::vector<int> used_in(size_t(din) * p.n_orbits, 0), used_out(size_t(dout) * p.n_orbits, 0);
-  std::vector<double> partial(size_t(nb) * dd, 0.0), sx(kGradBigOrbits * kGradBigMaxSide),
-      sy(kGradBigOrbits * kGradBigMaxSide);
-  QSV_CHECK_ARG(dd <= kGradBigPerThread * kBlock, "big gradient: too many entries");
+  std::vector<double> partial(size_t(nb) * dd, 0.0);
   for (int blk = 0; blk < nb; ++blk) {
-    std::vector<double> acc(dd, 0.0);
+    std::vector<double> acc(size_t(tiles) * 64 * 4, 0.0);
     for (uint32_t c = blk; c < nchunks; c += nb) {
-      for (int f = 0; f < kGradBigOrbits * din; ++f) {
-        const int ol = f / din, i = f - ol * din;
-        const uint32_t m = c * kGradBigOrbits + ol;
-        double v = 0.0;
-        if (m < p.n_orbits) {
+      std::vector<double> sm(kLds, 0.0);
+      auto stage = [&](bool out_side) -> int {
+        const int d = out_side ? dout : din, row = out_side ? ry : rx;
+        for (int f = 0; f < NO * d; ++f) {
+          const int ol = along ? f / d : f & (NO - 1), e = along ? f - ol * d : f / NO;
+          const uint32_t m = c * NO + ol;
           int64_t bin, bout;
-          orbit_base(p.g, m, bin, bout);
-          const int64_t a = bin + oin[i];
-          QSV_CHECK_ARG(a >= 0 && a < p.n_in, "big gradient: x load out of bounds");
-          v = x[a];
-          ++used_in[size_t(i) * p.n_orbits + m];
+          orbit_base(p.g, m < p.n_orbits ? m : p.n_orbits - 1, bin, bout);
+          const int64_t a = out_side
+                                ? bout + big_offset(p.bg.k, p.bg.dout_t, p.bg.sout_t, e)
+                                : bin + big_offset(p.bg.k, p.bg.din_t, p.bg.sin_t, e);
+          const int slot = (out_side ? NO * rx : 0) + ol * row + e;
+          QSV_CHECK_ARG(slot < kLds, "big gradient: LDS slot %d", slot);
+          if (m >= p.n_orbits) continue;
+          QSV_CHECK_ARG(a >= 0 && a < (out_side ? p.n_out : p.n_in),
+                        "big gradient: load out of bounds");
+          sm[slot] = out_side ? ybar[a] : x[a];
+          ++(out_side ? used_out : used_in)[size_t(e) * p.n_orbits + m];
         }
-        sx[ol * kGradBigMaxSide + i] = v;
-      }
-      for (int f = 0; f < kGradBigOrbits * dout; ++f) {
-        const int ol = f / dout, o = f - ol * dout;
-        const uint32_t m = c * kGradBigOrbits + ol;
-        double v = 0.0;
-        if (m < p.n_orbits) {
-          int64_t bin, bout;
-          orbit_base(p.g, m, bin, bout);
-          const int64_t a = bout + oout[o];
-          QSV_CHECK_ARG(a >= 0 && a < p.n_out, "big gradient: ybar load out of bounds");
-          v = ybar[a];
-          ++used_out[size_t(o) * p.n_orbits + m];
-        }
-        sy[ol * kGradBigMaxSide + o] = v;
-      }
-      for (int j = 0; j < dd; ++j) {
-        const int o = j / din, i = j - o * din;
-        for (int ol = 0; ol < kGradBigOrbits; ++ol)
-          acc[j] += sy[ol * kGradBigMaxSide + o] * sx[ol * kGradBigMaxSide + i];
-      }
+        return QSV_OK;
+      };
+      if (stage(false) || stage(true)) return QSV_EINVAL;
+      for (int t = 0; t < tiles; ++t)
+        for (int s = 0; s < NO / 4; ++s)
+          for (int lane = 0; lane < 64; ++lane)
+            for (int q = 0; q < 4; ++q) {
+              const int row = 16 * (t / ct) + (lane >> 4) + 4 * q, col = 16 * (t % ct) + (lane & 15);
+              for (int kk = 0; kk < 4; ++kk) {
+                const int ia = NO * rx + (4 * s + kk) * ry + row, ib = (4 * s + kk) * rx + col;
+                QSV_CHECK_ARG(ia < kLds && ib < kLds, "big gradient: LDS read");
+                acc[(size_t(t) * 64 + lane) * 4 + q] += sm[ia] * sm[ib];
+              }
+            }
     }
-    for (int j = 0; j < dd; ++j) partial[size_t(blk) * dd + j] = acc[j];
+    for (int t = 0; t < tiles; ++t)
+      for (int lane = 0; lane < 64; ++lane)
+        for (int q = 0; q < 4; ++q) {
+          const int o = 16 * (t / ct) + (lane >> 4) + 4 * q, i = 16 * (t % ct) + (lane & 15);
+          if (o < dout && i < din)
+            partial[size_t(blk) * dd + o * din + i] = acc[(size_t(t) * 64 + lane) * 4 + q];
+        }
   }
   for (size_t j = 0; j < used_in.size(); ++j)
     QSV_CHECK_ARG(used_in[j] == 1, "big gradient: x entry staged %d times", used_in[j]);
