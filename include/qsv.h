@@ -289,6 +289,23 @@ int qsv_emulate_window_blocks(int n_pos, const qsv_wblock* table, int batch, int
                               int64_t out_elems, const double* dout, double* drot,
                               double* ddamp_part);
 
+/* The same blocks for one window over all `layers` layers (f_layer in
+ * [0, layers)): the blocks of any fusion plan of the layered circuit, each
+ * gate in one block; ddamp_part is [batch][layers][n_qubits][4][4]. */
+int qsv_layer_blocks(int dtype, int n_pos, const qsv_wblock* table_host,
+                     const qsv_wblock* table_dev, int batch, int n_qubits, int layers,
+                     const double* rot, const double* damp, const double* cz, void* out,
+                     int64_t out_elems, void* stream);
+int qsv_layer_blocks_backward(int dtype, int n_pos, const qsv_wblock* table_host,
+                              const qsv_wblock* table_dev, int batch, int n_qubits, int layers,
+                              const double* rot, const double* damp, const double* cz,
+                              const void* dout, int64_t out_elems, double* drot,
+                              double* ddamp_part, void* stream);
+int qsv_emulate_layer_blocks(int n_pos, const qsv_wblock* table, int batch, int n_qubits,
+                             int layers, const double* rot, const double* damp, const double* cz,
+                             double* out, int64_t out_elems, const double* dout, double* drot,
+                             double* ddamp_part);
+
 /* Bytes of device workspace qsv_ptm_grad / qsv_ptm_grad_tiled need (enough
  * for any launch shape). */
 int64_t qsv_ptm_grad_workspace_bytes(int batch, int rank, const int64_t* dims, int k,

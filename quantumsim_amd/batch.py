@@ -4,9 +4,9 @@ Narrow circuits (up to ``persistent.max_qubits()`` qubits, 7 in float32 on
 MI355X) all run in ONE persistent kernel launch (forward) and one more
 (adjoint): a workgroup per circuit, its Pauli vector in LDS, every width and
 depth in the same launch (quantumsim_amd/persistent.py).  The PTMs of all
-their gates are computed by torch from the circuit parameters in a handful
-of batched ops (all layers of a parity at once) into one pool, so autograd
-carries dL/dP from the adjoint kernel to the angles and T1/T2.
+their gates are built from the circuit parameters by one launch per width
+(windows.LayerGatePlan) into one pool, and one more maps dL/dP from the
+adjoint kernel back towards the angles and T1/T2.
 
 Wider circuits (whose states, 256 KB to 16 MB each, do not fit in LDS and
 are streamed at HBM bandwidth anyway) are grouped by qubit count; inside a
@@ -47,7 +47,7 @@ from .bases import general
 from .fusion import fuse_batched, fuse_plan
 from .workloads import (rotation_ptms, damping_ptms, fused_layer_gates, layer_targets,
                         brickwork_window_plan)
-from .windows import WindowPlan, window_blocks
+from .windows import LayerGatePlan, WindowPlan, window_blocks
 
 __all__ = ['CircuitBatch', 'plain_forward_backward', 'choose_checkpoint_interval']
 
@@ -154,57 +154,57 @@ class CircuitBatch:
             checkpoint_every = choose_checkpoint_interval(self.kept_bytes, checkpoint_budget)
         self.k = max(1, int(checkpoint_every))
 
-    def _pool_layout(self):
-        """(group index, parity, gate index within the layer, D, layers of
-        that parity) of every piece of the PTM pool, in pool order."""
-        out = []
-        for gi in self.small:
-            g = self.groups[gi]
-            for p in (0, 1):
-                Lp = len(range(p, g.layers[0], 2))
-                if Lp == 0:
-                    continue
-                for j, t in enumerate(layer_targets(g.n, p)):
-                    out.append((gi, p, j, 4 ** len(t), Lp))
-        return out
+    def _pool_plan(self, gi):
+        """Gate plan of a narrow group: every gate of every two-layer window
+        (windows.LayerGatePlan); its output is the group's part of the PTM
+        pool, window-major per gate position."""
+        g = self.groups[gi]
+        plan = self._consts.get(('pool', gi))
+        if plan is None:
+            plan = LayerGatePlan(g.n, (g.layers[0] + 1) // 2, len(g.members), self.device)
+            shared_constant(plan.table_dev)
+            self._consts[('pool', gi)] = plan
+        return plan
 
     def _persistent_table(self):
-        base, off = {}, 0
-        for gi, p, j, D, Lp in self._pool_layout():
-            base[(gi, p, j)] = (off, Lp)
-            off += len(self.groups[gi].members) * Lp * D * D
+        off = 0
         circuits = []
         for gi in self.small:
             g = self.groups[gi]
-            targets = [layer_targets(g.n, p) for p in (0, 1)]
+            plan = self._pool_plan(gi)
+            B, n0 = len(g.members), len(layer_targets(g.n, 0))
+            by_parity = [plan.positions[:n0], plan.positions[n0:]]
             for b, L in enumerate(g.layers):
                 gates = []
                 for l in range(L):
-                    p, lp = l % 2, l // 2
-                    for j, t in enumerate(targets[p]):
-                        b0, Lp = base[(gi, p, j)]
-                        D = 4 ** len(t)
-                        gates.append((t, b0 + (b * Lp + lp) * D * D))
+                    for t, D, base in by_parity[l % 2]:
+                        gates.append((t, off + base + ((l // 2) * B + b) * D * D))
                 circuits.append((g.n, gates))
+            off += plan.out_elems
         return persistent.CircuitTable(circuits, off, device=self.device)
+
+    def _padded_rotations(self, g):
+        """Rotation PTMs [B, 2 nw, n, 4, 4] of group g's layers, padded to
+        whole two-layer windows."""
+        ang = g.angles
+        if ang.shape[1] % 2:
+            ang = torch.cat([ang, torch.zeros_like(ang[:, :1])], 1)
+        return rotation_ptms(ang)
 
     def _persistent_populations(self):
         """Populations of every narrow circuit: one forward launch over all
-        of them; per group [B, 2^n] in member order."""
+        of them; per group [B, 2^n] in member order.  The PTMs of all their
+        gates come from one launch per group (and one for the backward)."""
         pieces = []
+        cz = self._cached(('cz16',), lambda: cz_ptm(self.device).reshape(16, 16).contiguous())
         for gi in self.small:
             g = self.groups[gi]
-            B, n = len(g.members), g.n
-            rot = rotation_ptms(g.angles)            # [B, L, n, 4, 4]
-            damp = damping_ptms(g.t1, g.t2)          # [B, n, 4, 4]
-            for p in (0, 1):
-                Lp = len(range(p, g.layers[0], 2))
-                if Lp == 0:
-                    continue
-                rot_p = rot[:, p::2].reshape(B * Lp, n, 4, 4)
-                damp_p = damp[:, None].expand(B, Lp, n, 4, 4).reshape(B * Lp, n, 4, 4)
-                for gate in fused_layer_gates(n, p, rot_p, damp_p):
-                    pieces.append(gate.ptm.reshape(-1))
+            plan = self._pool_plan(gi)
+            keep8 = self._cached(('keepall', gi), lambda: torch.ones(
+                (plan.batch, plan.nw), dtype=torch.uint8, device=self.device))
+            gates = window_blocks(self._padded_rotations(g), damping_ptms(g.t1, g.t2), keep8,
+                                  plan, torch.float64, cz)
+            pieces += [m.reshape(-1) for m in gates]
         pool = torch.cat(pieces)
         pops = persistent.run(pool, self.ptable, self.dtype)
         out, pos = [], 0
@@ -261,10 +261,7 @@ class CircuitBatch:
         n, B = g.n, len(g.members)
         Lmax = g.layers[0]
         nw = (Lmax + 1) // 2
-        ang = g.angles
-        if 2 * nw > Lmax:                 # pad to whole windows (masked below)
-            ang = torch.cat([ang, torch.zeros_like(ang[:, :1])], 1)
-        rot = rotation_ptms(ang)                                  # [B, 2 nw, n, 4, 4]
+        rot = self._padded_rotations(g)                           # [B, 2 nw, n, 4, 4]
         damp = damping_ptms(g.t1, g.t2)                           # [B, n, 4, 4]
         if self.block_kernel and self.fuse_qudits == 3:
             # every block of every window and circuit in one launch (and one

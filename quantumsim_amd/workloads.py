@@ -265,6 +265,7 @@ class TrainableCircuit:
     def __init__(self, n=12, layers=40, block=5, n_blocks=3):
         self.n, self.layers, self.block, self.n_blocks = n, layers, block, n_blocks
         self.n_params = n_blocks * n * 2 + 2 * n
+        self._plans = {}           # block plans per (sets, device)
 
     def initial_params(self, sets, seed, device, dtype):
         import torch
@@ -291,6 +292,26 @@ class TrainableCircuit:
             out = [Gate(m, q) for m, q in fuse_batched(out, [4] * self.n, fuse_qudits)]
         return out
 
+    def _blocks(self, ang, t1, t2, dtype):
+        import torch
+        from .autograd import Gate, cz_ptm, shared_constant
+        from .windows import LayerBlockPlan, layer_blocks
+        key = (ang.shape[0], ang.device)
+        hit = self._plans.get(key)
+        if hit is None:
+            plan = LayerBlockPlan(self.n, self.layers, ang.shape[0], ang.device)
+            which = torch.tensor([(layer // self.block) % self.n_blocks
+                                  for layer in range(self.layers)], device=ang.device)
+            shared_constant(plan.table_dev)
+            hit = (plan, shared_constant(which))
+            if len(self._plans) >= 8:
+                self._plans.pop(next(iter(self._plans)))
+            self._plans[key] = hit
+        plan, which = hit
+        cz = cz_ptm(ang.device).reshape(16, 16).contiguous()
+        return [Gate(m, q) for m, q in layer_blocks(rotation_ptms(ang), damping_ptms(t1, t2),
+                                                    plan, dtype, cz, which)]
+
     def populations(self, ang, t1, t2, dtype, checkpoint_every=8, fuse_qudits=0):
         import torch
         from .autograd import run_circuit, diagonal
@@ -299,7 +320,11 @@ class TrainableCircuit:
         N = 4 ** self.n
         x0 = torch.zeros((S, N), dtype=dtype, device=ang.device)
         x0[:, 0] = 1
-        gates = self.gates(ang, t1, t2, fuse_qudits)
+        if fuse_qudits == 3 and ang.dtype == t1.dtype == t2.dtype == torch.float64:
+            # the blocks gates() composes, built by the library in one launch
+            gates = self._blocks(ang, t1, t2, dtype)
+        else:
+            gates = self.gates(ang, t1, t2, fuse_qudits)
         x = run_circuit(x0, gates, (4,) * self.n, checkpoint_every)
         return diagonal(x, [general(2)] * self.n)
 
