@@ -196,7 +196,7 @@ int64_t qsv_circuits_lds_bytes(int dtype, int max_qubits, int adjoint);
 /* One persistent launch runs every circuit of the table (widths up to
  * max_qubits <= qsv_circuits_max_qubits, any depths): each workgroup keeps a
  * circuit's Pauli vector in LDS, starts from |0..0><0..0|, applies the
- * gates with the pool's PTMs, writes the state before every gate to `traj`
+ * gates with the pool's PTMs, writes the state before every gate to `traj` (in an order private to the two entries)
  * and the float64 populations to `pops`.  Safe under HIP graph capture (one
  * kernel, tables and buffers in device memory).  No counterpart in the
  * reference (one circuit per PauliVector object there); used by the circuit
