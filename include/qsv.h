@@ -196,8 +196,9 @@ int64_t qsv_circuits_lds_bytes(int dtype, int max_qubits, int adjoint);
 /* One persistent launch runs every circuit of the table (widths up to
  * max_qubits <= qsv_circuits_max_qubits, any depths): each workgroup keeps a
  * circuit's Pauli vector in LDS, starts from |0..0><0..0|, applies the
- * gates with the pool's PTMs, writes the state before every gate to `traj` (in an order private to the two entries)
- * and the float64 populations to `pops`.  Safe under HIP graph capture (one
+ * gates with the pool's PTMs, writes the state before every gate to `traj`
+ * (in an order private to these two entries) and the float64 populations to
+ * `pops`.  Safe under HIP graph capture (one
  * kernel, tables and buffers in device memory).  No counterpart in the
  * reference (one circuit per PauliVector object there); used by the circuit
  * batcher for its narrow circuits. */
@@ -305,6 +306,25 @@ int qsv_emulate_layer_blocks(int n_pos, const qsv_wblock* table, int batch, int 
                              int layers, const double* rot, const double* damp, const double* cz,
                              double* out, int64_t out_elems, const double* dout, double* drot,
                              double* ddamp_part);
+
+/* The layered circuits' parameters in one launch (float64, general(2) basis):
+ * coef[batch][layers][n][9], coef[3 j + i] = f_j(b) f_i(a), f = (1, cos, sin),
+ * for angles [batch][own][n][(a, b)] (layers past `own`: angles 0), and
+ * damp[batch][n][4][4], amplitude then phase damping for a wait t under
+ * t1, t2 [batch][n].  The PTM of RZ(b) RX(a) is coef times its [9][16] terms.
+ * The backward gives dL/dangles, dL/dt1, dL/dt2 from dL/dPTM
+ * [batch][layers][n][16] and dL/ddamp in one launch.  Safe under HIP graph
+ * capture. */
+int qsv_gate_params(int batch, int layers, int own, int n, const double* angles, double* coef,
+                    const double* t1, const double* t2, double t, double* damp, void* stream);
+int qsv_gate_params_backward(int batch, int layers, int own, int n, const double* angles,
+                             const double* terms, const double* drot, double* dangles,
+                             const double* t1, const double* t2, double t, const double* ddamp,
+                             double* dt1, double* dt2, void* stream);
+int qsv_emulate_gate_params(int batch, int layers, int own, int n, const double* angles,
+                            const double* terms, double* coef, const double* t1,
+                            const double* t2, double t, double* damp, const double* drot,
+                            double* dangles, const double* ddamp, double* dt1, double* dt2);
 
 /* Bytes of device workspace qsv_ptm_grad / qsv_ptm_grad_tiled need (enough
  * for any launch shape). */

@@ -97,6 +97,12 @@ _SIGNATURES = {
                                                  ctypes.c_int, ctypes.c_int, _c_f64p, _c_f64p,
                                                  _vp, _c_f64p, _c_f64p, ctypes.c_int64, _c_f64p,
                                                  _c_f64p, _c_f64p]),
+    'qsv_gate_params': (ctypes.c_int, [ctypes.c_int] * 4 + [_vp] * 4 +
+                        [ctypes.c_double, _vp, _vp]),
+    'qsv_gate_params_backward': (ctypes.c_int, [ctypes.c_int] * 4 + [_vp] * 6 +
+                                 [ctypes.c_double] + [_vp] * 4),
+    'qsv_emulate_gate_params': (ctypes.c_int, [ctypes.c_int] * 4 + [_vp] * 5 + [ctypes.c_double] +
+                                [_vp] * 6),
     'qsv_layer_blocks': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _vp, _vp, ctypes.c_int,
                                         ctypes.c_int, ctypes.c_int, _vp, _vp, _vp, _vp,
                                         ctypes.c_int64, _vp]),

@@ -45,7 +45,7 @@ from .autograd import Gate, run_schedule, diagonal, shared_constant, cz_ptm
 from .autotune import tuning
 from .bases import general
 from .fusion import fuse_batched, fuse_plan
-from .workloads import (rotation_ptms, damping_ptms, fused_layer_gates, layer_targets,
+from .workloads import (gate_ptms, fused_layer_gates, layer_targets,
                         brickwork_window_plan)
 from .windows import LayerGatePlan, WindowPlan, window_blocks
 
@@ -183,13 +183,10 @@ class CircuitBatch:
             off += plan.out_elems
         return persistent.CircuitTable(circuits, off, device=self.device)
 
-    def _padded_rotations(self, g):
+    def _gate_ptms(self, g):
         """Rotation PTMs [B, 2 nw, n, 4, 4] of group g's layers, padded to
-        whole two-layer windows."""
-        ang = g.angles
-        if ang.shape[1] % 2:
-            ang = torch.cat([ang, torch.zeros_like(ang[:, :1])], 1)
-        return rotation_ptms(ang)
+        whole two-layer windows, and damping PTMs [B, n, 4, 4]."""
+        return gate_ptms(g.angles, g.t1, g.t2, (g.layers[0] + 1) // 2 * 2)
 
     def _persistent_populations(self):
         """Populations of every narrow circuit: one forward launch over all
@@ -202,8 +199,7 @@ class CircuitBatch:
             plan = self._pool_plan(gi)
             keep8 = self._cached(('keepall', gi), lambda: torch.ones(
                 (plan.batch, plan.nw), dtype=torch.uint8, device=self.device))
-            gates = window_blocks(self._padded_rotations(g), damping_ptms(g.t1, g.t2), keep8,
-                                  plan, torch.float64, cz)
+            gates = window_blocks(*self._gate_ptms(g), keep8, plan, torch.float64, cz)
             pieces += [m.reshape(-1) for m in gates]
         pool = torch.cat(pieces)
         pops = persistent.run(pool, self.ptable, self.dtype)
@@ -224,8 +220,7 @@ class CircuitBatch:
         ([layers of that parity, B, D, D] in the state's element type,
         targets); layer l is step l // 2 of parity l % 2."""
         n, B = g.n, len(g.members)
-        rot = rotation_ptms(g.angles)            # [B, L, n, 4, 4]
-        damp = damping_ptms(g.t1, g.t2)          # [B, n, 4, 4]
+        rot, damp = gate_ptms(g.angles, g.t1, g.t2)     # [B, L, n, 4, 4], [B, n, 4, 4]
         out = []
         for p in (0, 1):
             Lp = len(range(p, g.layers[0], 2))
@@ -261,8 +256,7 @@ class CircuitBatch:
         n, B = g.n, len(g.members)
         Lmax = g.layers[0]
         nw = (Lmax + 1) // 2
-        rot = self._padded_rotations(g)                           # [B, 2 nw, n, 4, 4]
-        damp = damping_ptms(g.t1, g.t2)                           # [B, n, 4, 4]
+        rot, damp = self._gate_ptms(g)           # [B, 2 nw, n, 4, 4], [B, n, 4, 4]
         if self.block_kernel and self.fuse_qudits == 3:
             # every block of every window and circuit in one launch (and one
             # for the backward): qsv_window_blocks

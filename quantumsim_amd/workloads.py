@@ -13,6 +13,8 @@ A circuit is a list of ``(ptm, qubits)`` with float64 PTMs in the
     (2,3), ... on even layers and (1,2), (3,4), ... on odd layers (14-qubit,
     60-layer case).
 """
+import functools
+
 import numpy as np
 
 from .algebra.algebra import kraus_to_ptm
@@ -252,6 +254,83 @@ def damping_ptms(t1, t2, t=GATE_TIME * 1e6):
     return p.reshape(*shp, 4, 4)
 
 
+def _gate_ptms_ops(angles, t1, t2, layers):
+    """gate_ptms by tensor operations."""
+    import torch
+    pad = layers - angles.shape[1]
+    if pad:
+        angles = torch.cat([angles, torch.zeros_like(angles[:, :1]).expand(
+            -1, pad, -1, -1)], 1)
+    return rotation_ptms(angles), damping_ptms(t1, t2)
+
+
+def gate_ptms(angles, t1, t2, layers=None):
+    """(rotation_ptms [B, layers, n, 4, 4], damping_ptms [B, n, 4, 4]) of
+    angles [B, L, n, 2] and t1, t2 [B, n]; layers beyond L have angles 0.
+    Float64 parameters on a device take one launch and the rotations' product
+    forward and one launch backward (the same values bit for bit as the
+    tensor operations', which take about 160 small launches), others the
+    tensor operations."""
+    import torch
+    layers = angles.shape[1] if layers is None else layers
+    if not (angles.is_cuda and angles.dtype == t1.dtype == t2.dtype == torch.float64
+            and angles.device == t1.device == t2.device and angles.dim() == 4
+            and angles.shape[3] == 2 and t1.shape == t2.shape == angles[:, 0, :, 0].shape):
+        return _gate_ptms_ops(angles, t1, t2, layers)
+    return _gate_ptms_function().apply(angles, t1, t2, layers)
+
+
+@functools.lru_cache(maxsize=None)
+def _gate_ptms_function():
+    import torch
+    from . import _native as nat
+
+    def stream():
+        s = torch.cuda.current_stream().cuda_stream
+        return s if s else None
+
+    class GatePTMs(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, angles, t1, t2, layers):
+            ctx.save_for_backward(angles, t1, t2)
+            ctx.layers = layers
+            B, L, n, _ = angles.shape
+            a, p, q = (x.detach().contiguous() for x in (angles, t1, t2))
+            coef = torch.empty((B * layers * n, 9), dtype=a.dtype, device=a.device)
+            damp = torch.empty((B, n, 4, 4), dtype=a.dtype, device=a.device)
+            rc = nat.lib().qsv_gate_params(
+                B, layers, L, n, a.data_ptr(), coef.data_ptr(), p.data_ptr(), q.data_ptr(),
+                GATE_TIME * 1e6, damp.data_ptr(), stream())
+            nat.check(rc, 'gate_params')
+            rot = (coef @ _rotation_terms(a.device)).view(B, layers, n, 4, 4)
+            need = ctx.needs_input_grad
+            ctx.mark_non_differentiable(*([] if need[0] else [rot]),
+                                        *([] if need[1] or need[2] else [damp]))
+            return rot, damp
+
+        @staticmethod
+        def backward(ctx, drot, ddamp):
+            angles, t1, t2 = ctx.saved_tensors
+            if torch.is_grad_enabled():      # a gradient that is differentiated again
+                need = [x for x, w in zip((angles, t1, t2), ctx.needs_input_grad) if w]
+                pairs = [(o, g) for o, g in zip(_gate_ptms_ops(angles, t1, t2, ctx.layers),
+                                                (drot, ddamp)) if o.requires_grad]
+                out = iter(torch.autograd.grad([o for o, _ in pairs], need,
+                                               [g for _, g in pairs], create_graph=True))
+                return tuple(next(out) if w else None for w in ctx.needs_input_grad[:3]) + (None,)
+            B, L, n, _ = angles.shape
+            a, p, q, dr, dd = (x.contiguous() for x in (angles, t1, t2, drot, ddamp))
+            da, dp, dq = (torch.empty_like(x) for x in (a, p, q))
+            rc = nat.lib().qsv_gate_params_backward(
+                B, ctx.layers, L, n, a.data_ptr(), _rotation_terms(a.device).data_ptr(),
+                dr.data_ptr(), da.data_ptr(), p.data_ptr(), q.data_ptr(), GATE_TIME * 1e6,
+                dd.data_ptr(), dp.data_ptr(), dq.data_ptr(), stream())
+            nat.check(rc, 'gate_params_backward')
+            return da, dp, dq, None
+
+    return GatePTMs
+
+
 class TrainableCircuit:
     """12 qubits, 40 layers, 96 trainable parameters per parameter set:
     RX/RZ angles shared by the layers of a 5-layer block, three blocks used
@@ -309,8 +388,8 @@ class TrainableCircuit:
             self._plans[key] = hit
         plan, which = hit
         cz = cz_ptm(ang.device).reshape(16, 16).contiguous()
-        return [Gate(m, q) for m, q in layer_blocks(rotation_ptms(ang), damping_ptms(t1, t2),
-                                                    plan, dtype, cz, which)]
+        return [Gate(m, q) for m, q in layer_blocks(*gate_ptms(ang, t1, t2), plan, dtype, cz,
+                                                    which)]
 
     def populations(self, ang, t1, t2, dtype, checkpoint_every=8, fuse_qudits=0):
         import torch
