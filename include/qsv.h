@@ -393,6 +393,52 @@ int qsv_apply_ptm_batched_backward(int dtype, const void* x, const void* ybar, v
                                    int64_t ptm_batch_stride, void* dptm, int accumulate,
                                    void* workspace, int64_t workspace_bytes, void* stream);
 
+/* QSV_OK if qsv_apply_ptm_batched_backward takes this geometry (its states
+ * aligned), QSV_ENOTSUP if not. */
+int qsv_batched_backward_applies(int dtype, int rank, const int64_t* dims, int k,
+                                 const int32_t* targets);
+
+/* One segment of a gate schedule (`active` states back to back, square PTMs):
+ * the launches of its gates, in order, from one call.  A gate is a pair
+ * (position p, step w); the PTMs of step w are at ptm + w * step elements, one
+ * per state `state` elements apart (0: one for all).
+ *   forward:  x -> outs[0] -> outs[1] ... (one output per gate).
+ *   backward: from the last gate to the first, dL/dx of every gate into the other
+ *     of bufs[2] (bufs[cur] holds dL/d(last output); *cur_out: where dL/dx
+ *     of the first gate is) and dL/dP at grad_ptm + w * step (NULL: not
+ *     wanted).  kept[c]: the state before gate c * every; the states between
+ *     are applied again into between[every - 1].  `fused` positions with
+ *     aligned states take qsv_apply_ptm_batched_backward, others
+ *     qsv_ptm_grad_tiled and the apply with ptm_t, the transposed PTMs.
+ *     workspace: at least every position's `workspace` bytes (what
+ *     qsv_ptm_grad_workspace_bytes gives for `active`); with more, the final
+ *     sums of up to sixteen gradients share a launch (without a hook).
+ * hook (may be NULL): called before (phase 0) and after (phase 1) each launch
+ * with its kind, position and batch.  Same launches as the single calls;
+ * safe under HIP graph capture. */
+#define QSV_SCHED_APPLY 0
+#define QSV_SCHED_GRAD 1
+#define QSV_SCHED_BACKWARD 2
+typedef void (*qsv_sched_hook)(int phase, int kind, int pos, int batch);
+typedef struct qsv_sched_pos {
+  int32_t k, n_steps, fused, has_apply, has_grad, reserved;
+  int32_t targets[QSV_MAX_TARGETS];
+  qsv_tile apply, grad; /* launch shapes, where has_* */
+  const void *ptm, *ptm_t;
+  void* grad_ptm;
+  int64_t step, state, workspace;
+} qsv_sched_pos;
+int qsv_schedule_forward(int dtype, int rank, const int64_t* dims, int n_pos,
+                         const qsv_sched_pos* pos, int active, int n_gates,
+                         const int32_t* gates, const void* x, void* const* outs,
+                         qsv_sched_hook hook, void* stream);
+int qsv_schedule_backward(int dtype, int rank, const int64_t* dims, int n_pos,
+                          const qsv_sched_pos* pos, int active, int n_gates,
+                          const int32_t* gates, int every, const void* const* kept,
+                          void* const* between, void* const* bufs, int cur, void* workspace,
+                          int64_t workspace_bytes, int* cur_out, qsv_sched_hook hook,
+                          void* stream);
+
 /* qsv_ptm_grad with an explicit launch shape (tile->grad_blocks, at most 64
  * for PTMs above 16 x 16; NULL = automatic).  The result does not depend on
  * the shape beyond the order of the partial sums. */

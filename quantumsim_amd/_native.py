@@ -40,6 +40,19 @@ class Tile(ctypes.Structure):
         return (self.kernel, self.tile_orbits, self.grad_blocks)
 
 
+class SchedPos(ctypes.Structure):
+    """qsv_sched_pos (include/qsv.h): a gate position of a schedule."""
+    _fields_ = ([(n, ctypes.c_int32) for n in ('k', 'n_steps', 'fused', 'has_apply', 'has_grad',
+                                               'reserved')] +
+                [('targets', ctypes.c_int32 * 8), ('apply', Tile), ('grad', Tile),
+                 ('ptm', ctypes.c_void_p), ('ptm_t', ctypes.c_void_p),
+                 ('grad_ptm', ctypes.c_void_p), ('step', ctypes.c_int64),
+                 ('state', ctypes.c_int64), ('workspace', ctypes.c_int64)])
+
+
+SCHED_APPLY, SCHED_GRAD, SCHED_BACKWARD = 0, 1, 2
+SchedHook = ctypes.CFUNCTYPE(None, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int)
+
 KERNEL_AUTO, KERNEL_DIRECT, KERNEL_LDS = 0, 1, 2
 _vp = ctypes.c_void_p
 
@@ -75,6 +88,15 @@ _SIGNATURES = {
     'qsv_emulate_ptm_grad': (ctypes.c_int, [ctypes.c_int, _c_f64p, _c_f64p, ctypes.c_int, _c_i64p,
                                             ctypes.c_int, _c_i32p, _c_i32p, _c_f64p,
                                             ctypes.c_int32, _c_i32p]),
+    'qsv_batched_backward_applies': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _c_i64p,
+                                                    ctypes.c_int, _c_i32p]),
+    'qsv_schedule_forward': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _c_i64p, ctypes.c_int,
+                                            _vp, ctypes.c_int, ctypes.c_int, _vp, _vp, _vp,
+                                            SchedHook, _vp]),
+    'qsv_schedule_backward': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _c_i64p, ctypes.c_int,
+                                             _vp, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_int,
+                                             _vp, _vp, _vp, ctypes.c_int, _vp, ctypes.c_int64,
+                                             _c_i32p, SchedHook, _vp]),
     'qsv_apply_ptm_batched_backward': (ctypes.c_int, [ctypes.c_int, _vp, _vp, _vp, ctypes.c_int,
                                                       ctypes.c_int, _c_i64p, ctypes.c_int,
                                                       _c_i32p, _vp, ctypes.c_int64, _vp,

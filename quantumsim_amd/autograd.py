@@ -48,8 +48,9 @@ class _Workspace:
     _bufs = {}
 
     @classmethod
-    def get(cls, device, nbytes):
-        key = (device, torch.cuda.current_stream(device).cuda_stream)
+    def get(cls, device, nbytes, use=None):
+        """``use``: a purpose with a buffer of its own."""
+        key = (device, torch.cuda.current_stream(device).cuda_stream, use)
         t = cls._bufs.get(key)
         if t is None or t.numel() < nbytes:
             t = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
@@ -314,26 +315,121 @@ def run_circuit(x0, gates, shape, checkpoint_every=8):
     return _Circuit.apply(x0, meta, *ptms)
 
 
+# Partial sums of a schedule's PTM gradients kept per stream: sixteen gates of
+# six 8-qubit circuits (25 MB) or five of six 11-qubit ones, and the partials are
+# still in the 256 MB last-level cache when they are summed.  A fixed size, so that
+# the buffer a captured graph holds is replaced only for a larger single gate.
+_SCHEDULE_SCRATCH = 64 << 20
+
+
+class _SchedulePositions:
+    """The gate positions of a schedule as the library takes them
+    (qsv_sched_pos), for one pass: steps [n_steps, B, D, D] per position,
+    transposed and gradient tensors where the backward has them."""
+
+    def __init__(self, shape, targets, steps, grads=None, transposed=None, fused=None):
+        self.shape, self.targets, self.steps = shape, targets, steps
+        self.dims = [[shape[q] for q in t] for t in targets]
+        self.grads = grads
+        self.refs = transposed                       # keeps the copies alive
+        self.rows = (nat.SchedPos * max(len(steps), 1))()
+        for p, (r, t, tg) in enumerate(zip(self.rows, steps, targets)):
+            D = t.shape[-1]
+            r.k, r.n_steps, r.targets[:len(tg)] = len(tg), t.shape[0], tg
+            r.ptm, r.step = t.data_ptr(), t.shape[1] * D * D
+            r.state = 0 if t.shape[1] == 1 else D * D
+            if grads is not None:
+                r.fused = bool(fused[p])
+                r.ptm_t = transposed[p].data_ptr() if transposed[p] is not None else None
+                r.grad_ptm = grads[p].data_ptr() if grads[p] is not None else None
+
+    def for_batch(self, dtype, active, used):
+        """Launch shapes (and gradient scratch) of the positions ``used`` for
+        ``active`` states; returns the scratch bytes."""
+        tuner, L, most = get_tuner(), nat.lib(), 0
+        for p in used:
+            r, tg, d = self.rows[p], self.targets[p], self.dims[p]
+            tile = tuner.apply_tile(dtype, active, self.shape, tg, d)
+            r.has_apply = tile is not None
+            if tile is not None:
+                r.apply = tile
+            if self.grads is not None and self.grads[p] is not None:
+                tile = tuner.grad_tile(dtype, active, self.shape, tg, d)
+                r.has_grad = tile is not None
+                if tile is not None:
+                    r.grad = tile
+                r.workspace = nat.check(L.qsv_ptm_grad_workspace_bytes(
+                    active, len(self.shape), nat.i64(self.shape), len(tg), nat.i32(tg),
+                    nat.i32(d)), 'ptm_grad')
+                most = max(most, r.workspace)
+        return most
+
+    def hook(self):
+        """Counts every launch in the ledger in force, if any."""
+        led = _ledger.active()
+        if led is None:
+            return nat.SchedHook()
+        N, es = math.prod(self.shape), self.steps[0].element_size()
+        events = []
+
+        def call(phase, kind, p, B):
+            if phase == 0:
+                events.append(led.begin())
+                return
+            ev, D, ptm = events.pop(), self.steps[p].shape[-1], self.steps[p][0].numel()
+            if kind == nat.SCHED_APPLY:
+                led.end(ev, _ledger.APPLY_DENSE64 if D == 64 else _ledger.APPLY_SMALL,
+                        es * (2 * B * N + ptm), 2 * 64 * B * N if D == 64 else 0)
+            elif kind == nat.SCHED_GRAD:
+                led.end(ev, _ledger.GRAD_DENSE64 if D > 16 else _ledger.GRAD_SMALL,
+                        es * B * (2 * N + D * D), 2 * B * N * D if D > 16 else 0)
+            else:
+                led.end(ev, _ledger.BWD_DENSE64, es * (B * (3 * N + 64 * 64) + ptm),
+                        2 * 64 * B * 2 * N)
+        return nat.SchedHook(call)
+
+
+def _pointers(tensors):
+    return (nat.ctypes.c_void_p * max(len(tensors), 1))(*[t.data_ptr() for t in tensors])
+
+
 class _Schedule(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x0, meta, *steps):
         shape, targets, segments, k = meta
-        dims = [[shape[q] for q in t] for t in targets]
+        L, code, dims = nat.lib(), nat.dtype_code(x0.dtype), nat.i64(shape)
         finals = torch.empty_like(x0)
+        pos = _SchedulePositions(shape, targets, steps)
+        hook = pos.hook()
         kept, cks = [], []
         x = x0
-        with torch.no_grad():
-            for active, nxt, gates in segments:
-                ck = [x]
-                for j, (pos, w) in enumerate(gates):
-                    x = _apply_raw(x, steps[pos][w], shape, targets[pos], dims[pos])
-                    if (j + 1) % k == 0 and j + 1 < len(gates):
-                        ck.append(x)
-                kept.append(len(ck))
-                cks += ck
-                if nxt < active:
-                    finals[nxt:active].copy_(x[nxt:])
-                x = x[:nxt]
+        for active, nxt, gates, used in segments:
+            G = len(gates)
+            ck = [x]
+            outs, between = [], {}
+            for j in range(G):
+                # kept: checkpoints and the segment's last state; the others
+                # alternate between two buffers
+                if (j + 1) % k == 0 or j + 1 == G:
+                    y = x0.new_empty((active, x0.shape[1]))
+                    if j + 1 < G:
+                        ck.append(y)
+                else:
+                    y = between.get(j % 2)
+                    if y is None:
+                        y = between[j % 2] = x0.new_empty((active, x0.shape[1]))
+                outs.append(y)
+            if G:
+                pos.for_batch(x0.dtype, active, used)
+                nat.check(L.qsv_schedule_forward(
+                    code, len(shape), dims, len(steps), pos.rows, active, G, gates.ctypes.data,
+                    x.data_ptr(), _pointers(outs), hook, _stream()), 'schedule_forward')
+                x = outs[-1]
+            kept.append(len(ck))
+            cks += ck
+            if nxt < active:
+                finals[nxt:active].copy_(x[nxt:])
+            x = x[:nxt]
         ctx.meta = meta
         ctx.kept = kept
         ctx.save_for_backward(*cks, *steps)
@@ -342,7 +438,7 @@ class _Schedule(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gf):
         shape, targets, segments, k = ctx.meta
-        dims = [[shape[q] for q in t] for t in targets]
+        L, code, dims = nat.lib(), nat.dtype_code(gf.dtype), nat.i64(shape)
         saved = ctx.saved_tensors
         n_ck = sum(ctx.kept)
         cks, steps = saved[:n_ck], saved[n_ck:]
@@ -351,49 +447,44 @@ class _Schedule(torch.autograd.Function):
         # every (position, step) PTM is used by exactly one gate: its rows
         # of the running prefix are written in place, the rest stay zero
         grads = [torch.zeros_like(t) if nd else None for t, nd in zip(steps, need)]
-        # transposed PTMs for the adjoint applies, one copy per position that
-        # needs them (float32 64 x 64 blocks run the one-pass backward)
-        steps_t = {}
-
-        def transposed(pos):
-            if pos not in steps_t:
-                steps_t[pos] = steps[pos].transpose(-1, -2).contiguous()
-            return steps_t[pos]
-        fused = gf.dtype == torch.float32
+        # float32 64 x 64 blocks run the one-pass backward where the library
+        # has it; the others need transposed PTMs for the adjoint applies, one
+        # copy per position
+        fused, transposed = [], []
+        aligned = all(t.data_ptr() % 16 == 0 for t in cks)
+        for t, tg, g in zip(steps, targets, grads):
+            one = False
+            if gf.dtype == torch.float32 and g is not None and t.shape[-1] == 64:
+                rc = L.qsv_batched_backward_applies(code, len(shape), dims, len(tg), nat.i32(tg))
+                one = rc == 0
+                if rc != -3:                   # -3: the separate kernels
+                    nat.check(rc, 'backward')
+            fused.append(one)
+            transposed.append(None if one and aligned
+                              else t.transpose(-1, -2).contiguous())
+        pos = _SchedulePositions(shape, targets, steps, grads, transposed, fused)
+        hook = pos.hook()
         bufs = [torch.empty_like(gf), torch.empty_like(gf)]
-        cur = 0
+        cur = nat.ctypes.c_int32(0)
         base = n_ck
         for si in reversed(range(len(segments))):
-            active, nxt, gates = segments[si]
+            active, nxt, gates, used = segments[si]
             base -= ctx.kept[si]
             ck = cks[base:base + ctx.kept[si]]
             # adjoint of the segment's output: the continuing rows are in
             # place from the later segments; the finished rows come from gf
             if nxt < active:
-                bufs[cur][nxt:active].copy_(gf[nxt:active])
+                bufs[cur.value][nxt:active].copy_(gf[nxt:active])
             G = len(gates)
-            for c in reversed(range(len(ck))):
-                lo, hi = c * k, min(G, (c + 1) * k)
-                xs = [ck[c]]
-                for j in range(lo, hi - 1):
-                    pos, w = gates[j]
-                    xs.append(_apply_raw(xs[-1], steps[pos][w], shape, targets[pos], dims[pos]))
-                for j in reversed(range(lo, hi)):
-                    pos, w = gates[j]
-                    gy = bufs[cur][:active]
-                    done = None
-                    if fused and grads[pos] is not None:
-                        done = _fused_backward_raw(xs[j - lo], gy, steps[pos][w], shape,
-                                                   targets[pos], gx_out=bufs[1 - cur][:active],
-                                                   gp_out=grads[pos][w])
-                    if done is None:
-                        if grads[pos] is not None:
-                            _ptm_grad_raw(xs[j - lo], gy, shape, targets[pos], dims[pos],
-                                          out=grads[pos][w])
-                        _apply_raw(gy, transposed(pos)[w], shape, targets[pos], dims[pos],
-                                   out=bufs[1 - cur][:active])
-                    cur = 1 - cur
-        gx = bufs[cur] if ctx.needs_input_grad[0] else None
+            if G:
+                ws = _Workspace.get(gf.device, max(_SCHEDULE_SCRATCH, pos.for_batch(
+                    gf.dtype, active, used)), 'schedule')
+                between = [gf.new_empty((active, gf.shape[1])) for _ in range(min(k, G) - 1)]
+                nat.check(L.qsv_schedule_backward(
+                    code, len(shape), dims, len(steps), pos.rows, active, G, gates.ctypes.data, k,
+                    _pointers(ck), _pointers(between), _pointers(bufs), cur.value, ws.data_ptr(), ws.numel(),
+                    nat.ctypes.byref(cur), hook, _stream()), 'schedule_backward')
+        gx = bufs[cur.value] if ctx.needs_input_grad[0] else None
         return (gx, None, *grads)
 
 
@@ -432,22 +523,27 @@ def run_schedule(x0, steps, targets, segments, shape, checkpoint_every=1):
     # the running prefix starts with every state, shrinks from segment to
     # segment and ends empty, so every state's final value is written once
     prev = B
-    seen = set()
+    n_steps = np.array([t.shape[0] for t in steps], dtype=np.int64)
+    total, parts, seen = int(n_steps.sum()), [], []
     for active, cont, gates in segments:
         if active != prev or not 0 <= cont <= active:
             raise ValueError('segments must start with all {} states and hand each '
                              'segment the previous one\'s continuing states'.format(B))
         prev = cont
-        for p, w in gates:
-            if not (0 <= p < len(steps) and 0 <= w < steps[p].shape[0]):
-                raise ValueError('gate ({}, {}) outside the steps tensors'.format(p, w))
-            if (p, w) in seen:
-                raise ValueError('each (position, step) PTM drives one gate')
-            seen.add((p, w))
+        gs = np.ascontiguousarray(np.array(gates, dtype=np.int32).reshape(-1, 2))
+        bad = (gs < 0).any(1) | (gs[:, 0] >= len(steps))
+        if not bad.any():
+            bad = gs[:, 1] >= n_steps[gs[:, 0]]
+        if bad.any():
+            raise ValueError('gate ({}, {}) outside the steps tensors'.format(
+                *gs[int(np.argmax(bad))]))
+        seen.append(gs[:, 0] * np.int64(total + 1) + gs[:, 1])
+        parts.append((int(active), int(cont), gs, np.unique(gs[:, 0]).tolist()))
+    if seen and np.unique(np.concatenate(seen)).size != sum(len(s) for s in seen):
+        raise ValueError('each (position, step) PTM drives one gate')
     if prev != 0:
         raise ValueError('the last segment must leave no state running')
-    meta = (tuple(shape), [tuple(int(q) for q in t) for t in targets],
-            [(int(a), int(c), [(int(p), int(w)) for p, w in gs]) for a, c, gs in segments],
+    meta = (tuple(shape), [tuple(int(q) for q in t) for t in targets], parts,
             max(1, int(checkpoint_every)))
     return _Schedule.apply(x0, meta, *steps)
 

@@ -19,6 +19,7 @@
 // (deterministic).
 #include "qsv_fused.h"
 #include "qsv_geom.h"
+#include "qsv_grad.h"
 #include "qsv_lds.h"
 #include "qsv_mfma.h"
 
@@ -1119,18 +1120,22 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// One thread per (b, o, i): the block partials summed in order.  Sixteen loads
-// are in flight at a time: one after the other, a thread's 64 partials took
-// 13 us (their latencies) on a few blocks of the chip; 4.2 us now.
+// One thread per (gradient, b, o, i): the block partials summed in order.  Sixteen
+// loads are in flight at a time: one after the other, a thread's 64 partials took
+// 13 us (their latencies) on a few blocks of the chip; 4.2 us now.  A schedule's
+// backward sums up to sixteen gradients a launch (a sum by itself is a few
+// dozen blocks for 256 compute units and a launch between two larger ones).
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    k_ptm_grad_final(const double* __restrict__ partial, int nblocks, int dd,
-                     T* __restrict__ out, double scale_out_accumulate) {
+    k_ptm_grad_final(const GradFinals finals, double scale_out_accumulate) {
   constexpr int U = 16;
+  const GradFinal& f = finals.it[blockIdx.z];
+  const int dd = f.dd, nblocks = f.nb;
   const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   const int64_t b = blockIdx.y;
   if (j >= dd) return;
-  const double* p = partial + b * nblocks * dd + j;
+  T* out = static_cast<T*>(f.out);
+  const double* p = f.partial + b * nblocks * dd + j;
   double s = 0.0;
   int k = 0;
   for (; k + U <= nblocks; k += U) {
@@ -1150,6 +1155,32 @@ __global__ void __launch_bounds__(kBlock)
     out[b * dd + j] = T(double(out[b * dd + j]) + s);
   else
     out[b * dd + j] = T(s);
+}
+
+int launch_grad_finals(int dtype, const GradFinals& finals, int batch, int accumulate,
+                       hipStream_t s) {
+  if (finals.n == 0 || batch == 0) return QSV_OK;
+  int dd = 0;
+  for (int i = 0; i < finals.n; ++i) dd = std::max(dd, finals.it[i].dd);
+  const dim3 grid((dd + kBlock - 1) / kBlock, batch, finals.n);
+  const double acc_flag = accumulate ? 1.0 : 0.0;
+  if (dtype == QSV_F64)
+    hipLaunchKernelGGL(k_ptm_grad_final<double>, grid, dim3(kBlock), 0, s, finals, acc_flag);
+  else
+    hipLaunchKernelGGL(k_ptm_grad_final<float>, grid, dim3(kBlock), 0, s, finals, acc_flag);
+  QSV_CHECK_HIP(hipGetLastError());
+  return QSV_OK;
+}
+
+// The final sum of one gradient: appended to `defer`, or launched.
+static int grad_final(int dtype, const double* partial, int nb, int dd, void* out, int batch,
+                      int accumulate, GradFinals* defer, hipStream_t s) {
+  GradFinals one;
+  GradFinals& f = defer ? *defer : one;
+  if (!defer) one.n = 0;
+  QSV_CHECK_ARG(f.n < kGradFinals && !(defer && accumulate), "too many deferred gradient sums");
+  f.it[f.n++] = {partial, out, nb, dd};
+  return defer ? QSV_OK : launch_grad_finals(dtype, one, batch, accumulate, s);
 }
 
 struct GradPlan {
@@ -1628,8 +1659,8 @@ extern "C" int qsv_ptm_grad(int dtype, const void* x, const void* ybar, int batc
 static int ptm_grad_run(int dtype, const void* x, const void* ybar, int batch, int rank,
                         const int64_t* dims, int k, const int32_t* targets,
                         const int32_t* dims_out_t, void* dptm, int accumulate, void* partial_buf,
-                        int64_t partial_bytes, bool shrink, const qsv_tile* tile,
-                        void* stream) {
+                        int64_t partial_bytes, bool shrink, const qsv_tile* tile, void* stream,
+                        GradFinals* defer = nullptr) {
   QSV_CHECK_ARG(dtype == QSV_F32 || dtype == QSV_F64, "unknown dtype %d", dtype);
   QSV_CHECK_ARG(!tile || (tile->grad_blocks >= 0 && tile->grad_blocks <= kGradBlocks),
                 "tile: grad_blocks outside [0, %d]", kGradBlocks);
@@ -1666,18 +1697,19 @@ static int ptm_grad_run(int dtype, const void* x, const void* ybar, int batch, i
   else
     launch_grad<float>(p, vn, quad, grid, x, ybar, partial, s);
   QSV_CHECK_HIP(hipGetLastError());
-  const int dd = p.din * p.dout;
-  const dim3 g2((dd + kBlock - 1) / kBlock, batch);
-  const double acc_flag = accumulate ? 1.0 : 0.0;
-  if (dtype == QSV_F64)
-    hipLaunchKernelGGL(k_ptm_grad_final<double>, g2, dim3(kBlock), 0, s, partial, nb, dd,
-                       static_cast<double*>(dptm), acc_flag);
-  else
-    hipLaunchKernelGGL(k_ptm_grad_final<float>, g2, dim3(kBlock), 0, s, partial, nb, dd,
-                       static_cast<float*>(dptm), acc_flag);
-  QSV_CHECK_HIP(hipGetLastError());
-  return QSV_OK;
+  return grad_final(dtype, partial, nb, p.din * p.dout, dptm, batch, accumulate, defer, s);
 }
+
+namespace qsv {
+int ptm_grad_partials(int dtype, const void* x, const void* ybar, int batch, int rank,
+                      const int64_t* dims, int k, const int32_t* targets,
+                      const int32_t* dims_out_t, void* dptm, void* workspace,
+                      int64_t workspace_bytes, const qsv_tile* tile, GradFinals& finals,
+                      void* stream) {
+  return ptm_grad_run(dtype, x, ybar, batch, rank, dims, k, targets, dims_out_t, dptm, 0,
+                      workspace, workspace_bytes, false, tile, stream, &finals);
+}
+}  // namespace qsv
 
 extern "C" int qsv_ptm_grad_tiled(int dtype, const void* x, const void* ybar, int batch, int rank,
                                   const int64_t* dims, int k, const int32_t* targets,
@@ -2385,13 +2417,17 @@ static uint32_t bwd64_cap() {
   return cap;
 }
 
-extern "C" int qsv_apply_ptm_batched_backward(int dtype, const void* x, const void* ybar,
-                                              void* xbar, int batch, int rank,
-                                              const int64_t* dims, int k,
-                                              const int32_t* targets, const void* ptm_dev,
-                                              int64_t ptm_batch_stride, void* dptm,
-                                              int accumulate, void* workspace,
-                                              int64_t workspace_bytes, void* stream) {
+extern "C" int qsv_batched_backward_applies(int dtype, int rank, const int64_t* dims, int k,
+                                            const int32_t* targets) {
+  GradPlan p;
+  return bwd64_plan(dtype, rank, dims, k, targets, p);
+}
+
+static int batched_backward_run(int dtype, const void* x, const void* ybar, void* xbar, int batch,
+                                int rank, const int64_t* dims, int k, const int32_t* targets,
+                                const void* ptm_dev, int64_t ptm_batch_stride, void* dptm,
+                                int accumulate, void* workspace, int64_t workspace_bytes,
+                                void* stream, GradFinals* defer) {
   QSV_CHECK_ARG(batch >= 0 && batch <= 65535, "batch %d outside [0, 65535]", batch);
   QSV_CHECK_ARG(ptm_batch_stride >= 0, "negative PTM batch stride");
   GradPlan p;
@@ -2431,17 +2467,32 @@ extern "C" int qsv_apply_ptm_batched_backward(int dtype, const void* x, const vo
                        static_cast<double*>(xbar), p.g, p.n_orbits,
                        static_cast<const double*>(ptm_dev), ptm_batch_stride, p.offs, fo, partial);
   QSV_CHECK_HIP(hipGetLastError());
-  const dim3 g2((64 * 64 + kBlock - 1) / kBlock, batch);
-  const double acc_flag = accumulate ? 1.0 : 0.0;
-  if (dtype == QSV_F64)
-    hipLaunchKernelGGL(k_ptm_grad_final<double>, g2, dim3(kBlock), 0, s, partial, nb, 64 * 64,
-                       static_cast<double*>(dptm), acc_flag);
-  else
-    hipLaunchKernelGGL(k_ptm_grad_final<float>, g2, dim3(kBlock), 0, s, partial, nb, 64 * 64,
-                       static_cast<float*>(dptm), acc_flag);
-  QSV_CHECK_HIP(hipGetLastError());
-  return QSV_OK;
+  return grad_final(dtype, partial, nb, 64 * 64, dptm, batch, accumulate, defer, s);
 }
+
+extern "C" int qsv_apply_ptm_batched_backward(int dtype, const void* x, const void* ybar,
+                                              void* xbar, int batch, int rank,
+                                              const int64_t* dims, int k,
+                                              const int32_t* targets, const void* ptm_dev,
+                                              int64_t ptm_batch_stride, void* dptm,
+                                              int accumulate, void* workspace,
+                                              int64_t workspace_bytes, void* stream) {
+  return batched_backward_run(dtype, x, ybar, xbar, batch, rank, dims, k, targets, ptm_dev,
+                              ptm_batch_stride, dptm, accumulate, workspace, workspace_bytes,
+                              stream, nullptr);
+}
+
+namespace qsv {
+int batched_backward_partials(int dtype, const void* x, const void* ybar, void* xbar, int batch,
+                              int rank, const int64_t* dims, int k, const int32_t* targets,
+                              const void* ptm_dev, int64_t ptm_batch_stride, void* dptm,
+                              void* workspace, int64_t workspace_bytes, GradFinals& finals,
+                              void* stream) {
+  return batched_backward_run(dtype, x, ybar, xbar, batch, rank, dims, k, targets, ptm_dev,
+                              ptm_batch_stride, dptm, 0, workspace, workspace_bytes, stream,
+                              &finals);
+}
+}  // namespace qsv
 
 // Host replay of k_bwd64q + k_ptm_grad_final for one state: every direct
 // load (bounds, alignment, its four entries contiguous, its LDS slot),
