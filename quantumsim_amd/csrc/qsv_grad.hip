@@ -113,6 +113,7 @@ __global__ void __launch_bounds__(kBlock)
 // four waves' tiles are summed in float64 in LDS in a fixed order (32 KB),
 // one row block at a time, then the block writes its partial tile.
 constexpr int kGrad64Blocks = 64;
+constexpr int kBwdBlocks = 1024;  // blocks a float32 64 x 64 backward is split into at most
 constexpr int kGrad64Unroll = 1;
 // QUAD loads move 16 bytes of x and of ybar per lane and k-step (a quarter
 // of the orbit-vector mode's), so four k-steps are loaded before their
@@ -575,6 +576,22 @@ __device__ __forceinline__ void bwd_apply(const char* lds, const float (&pb)[16]
   *reinterpret_cast<f4*>(xbar + bin1 + xo) = v1;
 }
 
+// The tiles of one block of the float32 backward.  Block group i of `stride` takes
+// tiles i, i + stride, ...; its `parts` blocks take consecutive runs of `run` of
+// them, whole float32 partial sums (kDirFlush tiles), so that the same float32
+// sums are added in float64 however many blocks there are.
+struct BwdTiles {
+  uint32_t stride, parts, run;
+  __host__ __device__ void range(uint32_t block, uint32_t ntiles, uint32_t& t,
+                                 uint32_t& end) const {
+    const uint32_t j = block % parts;
+    const uint64_t first = block / parts + uint64_t(j) * run * stride;
+    const uint64_t last = first + uint64_t(run) * stride;
+    t = first < ntiles ? uint32_t(first) : ntiles;
+    end = parts > 1 && last < ntiles ? uint32_t(last) : ntiles;
+  }
+};
+
 // Fused float32 backward of a dense 64 x 64 block on k_ptm_grad64d's
 // staged tiles: per tile of 32 orbits, dP += ybar x^T (dir_compute, as in
 // k_ptm_grad64d) and xbar = P^T ybar from the same ybar tile in LDS
@@ -590,7 +607,7 @@ __global__ void __launch_bounds__(kBlock)
     k_bwd64d(const float* __restrict__ x, const float* __restrict__ ybar,
              float* __restrict__ xbar, const Geom g, const uint32_t n_orbits,
              const float* __restrict__ ptm, const int64_t pstride, const GradOffs offs,
-             double* __restrict__ partial) {
+             double* __restrict__ partial, const BwdTiles tiles) {
   __shared__ __align__(16) char st0[2 * kDirArr];
   __shared__ __align__(16) char st1[2 * kDirArr];
   const uint32_t b = blockIdx.y;
@@ -606,12 +623,16 @@ __global__ void __launch_bounds__(kBlock)
     oin[h] = offs.off_in[8 * (2 * w + h) + e];
     oout[h] = offs.off_out[8 * (2 * w + h) + e];
   }
+  const uint32_t stride = tiles.stride;
+  uint32_t t, ntiles;
+  tiles.range(blockIdx.x, n_orbits / kDirTile, t, ntiles);
+  if (t < ntiles) dir_issue<NT>(x, ybar, g, t, w, c, oin, oout, st0);
   const int n = lane & 15, kk = lane >> 4;
   const int64_t xo = offs.off_in[16 * w + n];
   float pb[16];
 #pragma unroll
   for (int s = 0; s < 16; ++s) pb[s] = ptm[(4 * s + kk) * 64 + 16 * w + n];
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the PTM, before any tile load
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the PTM (and the first tile)
   typedef Mfma<float>::acc Acc;
   Acc acc[4];
   double acc64[4][4];
@@ -629,10 +650,7 @@ __global__ void __launch_bounds__(kBlock)
       acc[cb] = Acc(0);
     }
   };
-  const uint32_t ntiles = n_orbits / kDirTile, stride = gridDim.x;
-  uint32_t t = blockIdx.x;
   int n_acc = 0;
-  if (t < ntiles) dir_issue<NT>(x, ybar, g, t, w, c, oin, oout, st0);
   while (t < ntiles) {
     const uint32_t t1 = t + stride;
     if (t1 < ntiles) {
@@ -793,7 +811,7 @@ __global__ void __launch_bounds__(kBlock)
     k_bwd64q(const float* __restrict__ x, const float* __restrict__ ybar,
              float* __restrict__ xbar, const Geom g, const uint32_t n_orbits,
              const float* __restrict__ ptm, const int64_t pstride, const GradOffs offs,
-             double* __restrict__ partial) {
+             double* __restrict__ partial, const BwdTiles tiles) {
   __shared__ __align__(16) char st0[2 * kQArr];
   __shared__ __align__(16) char st1[2 * kQArr];
   const uint32_t b = blockIdx.y;
@@ -803,6 +821,10 @@ __global__ void __launch_bounds__(kBlock)
   ptm += int64_t(b) * pstride;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t oiq = offs.off_in[4 * (lane >> 2)], ooq = offs.off_out[4 * (lane >> 2)];
+  const uint32_t stride = tiles.stride;
+  uint32_t t, ntiles;
+  tiles.range(blockIdx.x, n_orbits / kDirTile, t, ntiles);
+  if (t < ntiles) quad_issue<NT>(x, ybar, g, t, w, lane, oiq, ooq, st0);
   const int m = lane & 15, kk = lane >> 4;
   // A of the adjoint apply: P^T[16w + m][k] = P[k][16w + m], k-step s at
   // entry 16 (s / 4) + 4 kk + s % 4
@@ -811,7 +833,7 @@ __global__ void __launch_bounds__(kBlock)
   for (int sk = 0; sk < 16; ++sk)
     pa[sk] = ptm[(16 * (sk >> 2) + 4 * kk + (sk & 3)) * 64 + 16 * w + m];
   const int64_t xo = offs.off_in[16 * w + 4 * kk];
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the PTM, before any tile load
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the PTM (and the first tile)
   typedef Mfma<float>::acc Acc;
   Acc acc[4];
   double acc64[4][4];
@@ -829,10 +851,7 @@ __global__ void __launch_bounds__(kBlock)
       acc[cb] = Acc(0);
     }
   };
-  const uint32_t ntiles = n_orbits / kDirTile, stride = gridDim.x;
-  uint32_t t = blockIdx.x;
   int n_acc = 0;
-  if (t < ntiles) quad_issue<NT>(x, ybar, g, t, w, lane, oiq, ooq, st0);
   while (t < ntiles) {
     const uint32_t t1 = t + stride;
     if (t1 < ntiles) {
@@ -1595,7 +1614,9 @@ extern "C" int64_t qsv_ptm_grad_workspace_bytes(int batch, int rank, const int64
   GradPlan p;
   const int rc = make_grad_plan(8, rank, dims, k, targets, dims_out_t, p);
   if (rc) return rc;
-  return int64_t(batch) * max_grad_blocks(p) * p.din * p.dout * 8;
+  int64_t blocks = int64_t(batch) * max_grad_blocks(p);
+  if (p.din == 64 && p.dout == 64 && batch > 0) blocks = std::max<int64_t>(blocks, kBwdBlocks);
+  return blocks * p.din * p.dout * 8;
 }
 
 template <typename T>
@@ -1916,8 +1937,10 @@ static int emulate_grad64(const GradPlan& p, int es, const double* x, const doub
 // every MFMA operand read checked to find, in the stage of the current
 // tile, the (entry, orbit) the product needs; every entry of the partial
 // tiles written once.
-static int emulate_grad64d(const GradPlan& p, const double* x, const double* ybar, int nb,
-                           double* dptm, const double* ptm = nullptr, double* xbar = nullptr) {
+static int emulate_grad64d(const GradPlan& p, const double* x, const double* ybar,
+                           const BwdTiles& tiles, double* dptm, const double* ptm = nullptr,
+                           double* xbar = nullptr) {
+  const int nb = int(tiles.stride * tiles.parts);
   QSV_CHECK_ARG(grad64_direct(p, 4, p.vn), "grad64d: not a direct geometry");
   std::vector<int> xwritten(xbar ? size_t(p.n_in) : 0, 0);
   const uint32_t ntiles = p.n_orbits / kDirTile;
@@ -1930,7 +1953,8 @@ static int emulate_grad64d(const GradPlan& p, const double* x, const double* yba
   for (int blk = 0; blk < nb; ++blk) {
     std::vector<double> D(4 * 4 * 16 * 16, 0.0);  // [w][cb][row][col]
     int stage = 0;
-    for (uint32_t t = blk; t < ntiles; t += nb, stage ^= 1) {
+    uint32_t t, end;
+    for (tiles.range(blk, ntiles, t, end); t < end; t += tiles.stride, stage ^= 1) {
       double* sv = val.data() + size_t(stage) * nf;
       int64_t* stg = tag.data() + size_t(stage) * nf * 4;
       std::fill(stg, stg + size_t(nf) * 4, int64_t(-1));
@@ -2249,8 +2273,9 @@ extern "C" int qsv_emulate_ptm_grad(int dtype, const double* x, const double* yb
               (direct ? 2048 : 0);
   if (direct)
     return emulate_grad64d(p, x, ybar,
-                           grad_blocks_forced > 0 ? grad_blocks_forced
-                                                  : grad64_blocks(p.n_orbits, 1),
+                           {uint32_t(grad_blocks_forced > 0 ? grad_blocks_forced
+                                                            : grad64_blocks(p.n_orbits, 1)),
+                            1, 0},
                            dptm);
   if (p.big)
     return emulate_grad_big(p, x, ybar,
@@ -2382,21 +2407,34 @@ static int bwd64_blocks(const GradPlan& p, int batch, uint32_t cap) {
   return int(std::max<uint32_t>(nb, 1));
 }
 
-// k_bwd64d: one round of resident blocks over the batch (occupancy x CUs /
-// batch per state; measured on 8-12-qubit states: 5-12 % faster than the
-// gradient's 512 orbits per block), at least 4 tiles per block.
+// k_bwd64d / k_bwd64q: block groups, one round of resident blocks over the batch
+// (occupancy x CUs / batch per state), at least 4 tiles per group and at most
+// kGrad64Blocks.  A group is split (whole float32 partial sums each) until the
+// launch has kBwdBlocks blocks: two 11-qubit circuits make 128 groups for 256
+// compute units, and their training step took 12.5 ms, 8.0 ms with four blocks a
+// group; from six circuits (two blocks a group) on it makes no difference.
+static BwdTiles bwd64_split(uint32_t tiles, uint32_t stride, uint32_t batch) {
+  BwdTiles r;
+  r.stride = stride;
+  const uint32_t sums = ((tiles + stride - 1) / stride + kDirFlush - 1) / kDirFlush;
+  const uint32_t parts = std::max<uint32_t>(
+      1, std::min<uint32_t>(sums, kBwdBlocks / std::max<uint32_t>(1, stride * batch)));
+  const uint32_t each = std::max<uint32_t>(1, (sums + parts - 1) / parts);
+  r.parts = std::max<uint32_t>(1, (sums + each - 1) / each);
+  r.run = each * kDirFlush;
+  return r;
+}
 
-static int bwd64d_blocks(const GradPlan& p, int batch) {
+static BwdTiles bwd64_tiles(const GradPlan& p, int batch) {
   static const uint32_t cap_d =
       resident_blocks(reinterpret_cast<const void*>(k_bwd64d<true>));
   static const uint32_t cap_q =
       resident_blocks(reinterpret_cast<const void*>(k_bwd64q<true>));
-  const uint32_t cap = p.quad ? cap_q : cap_d;
+  const uint32_t cap = p.quad ? cap_q : cap_d, B = uint32_t(std::max(batch, 1));
   const uint32_t tiles = p.n_orbits / kDirTile;
-  uint32_t nb = cap / uint32_t(std::max(batch, 1));
-  nb = std::min(nb, tiles / 4);
-  nb = std::min<uint32_t>(nb, kGrad64Blocks);
-  return int(std::max<uint32_t>(nb, 1));
+  return bwd64_split(
+      tiles,
+      std::max<uint32_t>(1, std::min<uint32_t>(std::min(cap / B, tiles / 4), kGrad64Blocks)), B);
 }
 
 template <typename T, int VN>
@@ -2446,7 +2484,9 @@ static int batched_backward_run(int dtype, const void* x, const void* ybar, void
   const FusedOffs fo = bwd64_offsets(p);
   // bwd64_plan admits only k_bwd64d's and k_bwd64q's float32 geometries
   const bool direct = dtype == QSV_F32;
-  const int nb = direct ? bwd64d_blocks(p, batch) : bwd64_blocks(p, batch, bwd64_cap<double, 2>());
+  const BwdTiles tiles = direct ? bwd64_tiles(p, batch) : BwdTiles{1, 1, 1};
+  const int nb = direct ? int(tiles.stride * tiles.parts)
+                        : bwd64_blocks(p, batch, bwd64_cap<double, 2>());
   const int64_t need = int64_t(batch) * nb * 64 * 64 * 8;
   QSV_CHECK_ARG(workspace && workspace_bytes >= need, "fused backward needs %lld workspace bytes",
                 (long long)need);
@@ -2460,7 +2500,7 @@ static int batched_backward_run(int dtype, const void* x, const void* ybar, void
     hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, s, static_cast<const float*>(x),
                        static_cast<const float*>(ybar), static_cast<float*>(xbar), p.g,
                        p.n_orbits, static_cast<const float*>(ptm_dev), ptm_batch_stride, p.offs,
-                       partial);
+                       partial, tiles);
   } else
     hipLaunchKernelGGL((k_bwd64<double, 2>), grid, dim3(kBlock), 0, s,
                        static_cast<const double*>(x), static_cast<const double*>(ybar),
@@ -2499,8 +2539,9 @@ int batched_backward_partials(int dtype, const void* x, const void* ybar, void* 
 // every operand read of both contractions finding its (entry, orbit) in
 // the current stage, the MFMAs in hardware index order, every xbar store
 // in bounds and each xbar entry written once, each operand loaded once.
-static int emulate_bwd64q(const GradPlan& p, const double* x, const double* ybar, int nb,
-                          double* dptm, const double* ptm, double* xbar) {
+static int emulate_bwd64q(const GradPlan& p, const double* x, const double* ybar,
+                          const BwdTiles& tiles, double* dptm, const double* ptm, double* xbar) {
+  const int nb = int(tiles.stride * tiles.parts);
   QSV_CHECK_ARG(bwd64q_applies(p), "bwd64q: not a quad geometry");
   const uint32_t ntiles = p.n_orbits / kDirTile;
   const int nf = 2 * kQArr / 4;
@@ -2510,7 +2551,8 @@ static int emulate_bwd64q(const GradPlan& p, const double* x, const double* ybar
   std::vector<double> partial(size_t(nb) * 4096, 0.0);
   for (int blk = 0; blk < nb; ++blk) {
     std::vector<double> D(4 * 4 * 16 * 16, 0.0);  // [w][cb][row][col]
-    for (uint32_t t = blk; t < ntiles; t += nb) {
+    uint32_t t, end;
+    for (tiles.range(blk, ntiles, t, end); t < end; t += tiles.stride) {
       std::fill(stg.begin(), stg.end(), int64_t(-1));
       for (int w = 0; w < kBlock / 64; ++w)
         for (int lane = 0; lane < 64; ++lane) {
@@ -2770,9 +2812,11 @@ extern "C" int qsv_emulate_apply_ptm_batched_backward(int dtype, const double* x
                 kGrad64Blocks);
   const int es = dtype_size(dtype), VN = p.vn, MB = 4, KS = 16;
   if (dtype == QSV_F32) {  // bwd64_plan admits only k_bwd64d's and k_bwd64q's geometries
-    const int nbd = grad_blocks > 0 ? grad_blocks : grad64_blocks(p.n_orbits, 1);
-    return p.quad ? emulate_bwd64q(p, x, ybar, nbd, dptm, ptm, xbar)
-                  : emulate_grad64d(p, x, ybar, nbd, dptm, ptm, xbar);
+    const BwdTiles tiles = bwd64_split(
+        p.n_orbits / kDirTile,
+        uint32_t(grad_blocks > 0 ? grad_blocks : grad64_blocks(p.n_orbits, 1)), 1);
+    return p.quad ? emulate_bwd64q(p, x, ybar, tiles, dptm, ptm, xbar)
+                  : emulate_grad64d(p, x, ybar, tiles, dptm, ptm, xbar);
   }
   const int nb = grad_blocks > 0 ? grad_blocks : bwd64_blocks(p, 1, 256);
   const FusedOffs fo = bwd64_offsets(p);

@@ -4,7 +4,7 @@
 // of 10-50 us on the device; issued one library call at a time from the
 // interpreter they cost 13 us each on the host (allocation, views, argument
 // arrays), 28 of the step's 32 ms, with the device idle between them.  The same
-// calls in the same order from here cost @@.
+// calls in the same order from here cost 4-5 us each.
 //
 // Host code only: the entries it calls check their own arguments; the stream,
 // the buffers' sizes and the order of use are the caller's (one segment: `active`
