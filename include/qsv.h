@@ -556,6 +556,11 @@ int qsv_emulate_apply_ptm_batched_backward(int dtype, const double* x, const dou
 int qsv_emulate_apply_ptm_direct(int dtype, const double* x, double* y, int rank,
                                  const int64_t* dims, int k, const int32_t* targets,
                                  const double* ptm, int32_t blocks);
+/* The same for orbit vectors of four (k_apply64d: the innermost axis a
+ * bystander). */
+int qsv_emulate_apply_ptm_vectors(int dtype, const double* x, double* y, int rank,
+                                  const int64_t* dims, int k, const int32_t* targets,
+                                  const double* ptm, int32_t blocks);
 
 /* qsv_emulate_apply_ptm of the batched path's kernel choice for one state,
  * with an explicit launch shape (the autotuner's candidates are replayed

@@ -120,6 +120,11 @@ int launch_fused64_batched(int dtype, const FusedPlan& fp, const Geom& g, bool n
 // Float32 64 x 64 whose PTM's lowest index is the innermost axis (runs of
 // four entries) on whole 32-orbit tiles: the direct-to-LDS apply.
 bool apply64q_applies(int elem_bytes, const FusedPlan& fp);
+// Float32 64 x 64 on orbit vectors and whole 32-orbit tiles, one tile a block: batches
+// whose tiles are resident at once.
+bool apply64d_applies(int elem_bytes, const FusedPlan& fp, uint32_t batch);
+int launch_apply64d(const FusedPlan& fp, const Geom& g, bool nt, const void* in, void* out,
+                    const void* ptm_rows, int64_t pstride, uint32_t batch, hipStream_t s);
 int launch_apply64q(const FusedPlan& fp, const Geom& g, bool nt, const void* in, void* out,
                     const void* ptm_rows, int64_t pstride, uint32_t batch, hipStream_t s);
 

@@ -94,7 +94,22 @@ __global__ void __launch_bounds__(kBlock)
   in += int64_t(blockIdx.y) * g.bs_in;
   out += int64_t(blockIdx.y) * g.bs_out;
   pf += int64_t(blockIdx.y) * pstride;
-  if (prow) {
+  if (prow && sizeof(T) == 4) {
+    // wave w makes the fragments of row block w, a row per lane (row_operand,
+    // runs of four as they are): gathered one by one, each load touched sixteen
+    // cache lines (six states of 10 qubits 19.0 -> 16.8 us, of 11 qubits 49 -> 45)
+    const int ln = threadIdx.x & 63, w = threadIdx.x >> 6, jj = ln >> 4;
+    const T* row = pf + fused_frag_source(64, 4, VI, VO, w * 64 + (ln & 15));
+    float v[KS];
+    if constexpr (VI == 1) {
+      row_operand(reinterpret_cast<const float*>(row), jj, v);
+    } else {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) v[s] = row[16 * (s >> 2) + 4 * jj + (s & 3)];
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) As[(s * MB + w) * 64 + ln] = v[s];
+  } else if (prow) {
     for (int i = threadIdx.x; i < KS * MB * 64; i += kBlock)
       As[i] = pf[fused_frag_source(64, int(sizeof(T)), VI, VO, i)];
   } else {
@@ -400,6 +415,8 @@ int launch_fused64_batched(int dtype, const FusedPlan& fp, const Geom& g, bool n
   // faster than k_fused64<float, 4, 4, 1> on 8-12-qubit batches, same bits)
   if (dtype == QSV_F32 && apply64q_applies(4, fp))
     return launch_apply64q(fp, g, nt, in, out, ptm_rows, pstride, batch, s);
+  if (dtype == QSV_F32 && apply64d_applies(4, fp, batch))
+    return launch_apply64d(fp, g, nt, in, out, ptm_rows, pstride, batch, s);
   if (dtype == QSV_F64)
     return nt ? dispatch<double, 2, true>(fp, g, in, out, ptm_rows, s, batch, pstride, 1)
               : dispatch<double, 2, false>(fp, g, in, out, ptm_rows, s, batch, pstride, 1);

@@ -39,6 +39,29 @@ struct GradOffs {
   int64_t off_out[64];
 };
 
+// Entry offsets of a 64 x 64 PTM by index bit: the targets' dimensions multiply to
+// 64, so each is a run of the index's bits.  A lane adds up the ones it needs
+// (an array of them, indexed by lane, is read from the kernel arguments' memory by
+// every block: the float32 applies of 8-11 qubits took 0.1-1 us more, the
+// backwards 1-4 %).
+struct BitOffs {
+  int64_t in[6], out[6];
+};
+__host__ __device__ inline int64_t bit_off(const int64_t (&b)[6], uint32_t k) {
+  int64_t o = 0;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) o += (k >> i & 1) ? b[i] : 0;
+  return o;
+}
+static BitOffs bit_offs(const GradOffs& o) {
+  BitOffs r;
+  for (int i = 0; i < 6; ++i) {
+    r.in[i] = o.off_in[1 << i];
+    r.out[i] = o.off_out[1 << i];
+  }
+  return r;
+}
+
 template <typename T, int VN>
 __global__ void __launch_bounds__(kBlock)
     k_ptm_grad(const T* __restrict__ x, const T* __restrict__ ybar, const Geom g,
@@ -544,11 +567,13 @@ typedef float qsv_f2 __attribute__((ext_vector_type(2)));
 // B = P[4s + kk][16w + n] for all 16 k-steps in registers (pb).  Slot r of
 // lane l in row tile rt is orbit 8 (l / 16) + 2r + rt of entry 16w + l % 16,
 // so a lane ends with 8 consecutive orbits of one entry: two 16-byte stores.
-__device__ __forceinline__ void bwd_apply(const char* lds, const float (&pb)[16], int lane,
+// With P^T in place of P (and the output's strides, OUT) it is the forward apply.
+template <bool OUT>
+__device__ __forceinline__ void dir_apply(const char* arr, const float (&pb)[16], int lane,
                                           const Geom& g, uint32_t t, int64_t xo,
                                           float* __restrict__ xbar) {
   const int m = lane & 15, kk = lane >> 4;
-  const uint32_t ya = lds_off(lds + kDirArr + 16 * kk + 128 * (m >> 1) + 8 * (m & 1));
+  const uint32_t ya = lds_off(arr + 16 * kk + 128 * (m >> 1) + 8 * (m & 1));
   typedef Mfma<float>::acc Acc;
   Acc a0 = Acc(0), a1 = Acc(0);
   qsv_f2 av[8];
@@ -572,8 +597,8 @@ __device__ __forceinline__ void bwd_apply(const char* lds, const float (&pb)[16]
   f4 v0, v1;
   v0[0] = a0[0]; v0[1] = a1[0]; v0[2] = a0[1]; v0[3] = a1[1];
   v1[0] = a0[2]; v1[1] = a1[2]; v1[2] = a0[3]; v1[3] = a1[3];
-  *reinterpret_cast<f4*>(xbar + bin0 + xo) = v0;
-  *reinterpret_cast<f4*>(xbar + bin1 + xo) = v1;
+  *reinterpret_cast<f4*>(xbar + (OUT ? bout0 : bin0) + xo) = v0;
+  *reinterpret_cast<f4*>(xbar + (OUT ? bout1 : bin1) + xo) = v1;
 }
 
 // The tiles of one block of the float32 backward.  Block group i of `stride` takes
@@ -595,7 +620,7 @@ struct BwdTiles {
 // Fused float32 backward of a dense 64 x 64 block on k_ptm_grad64d's
 // staged tiles: per tile of 32 orbits, dP += ybar x^T (dir_compute, as in
 // k_ptm_grad64d) and xbar = P^T ybar from the same ybar tile in LDS
-// (bwd_apply), stored from the accumulators: x and ybar are read once, xbar
+// (dir_apply), stored from the accumulators: x and ybar are read once, xbar
 // written once (three streams where the transposed apply plus the gradient
 // move four).  The wait before each tile is vmcnt(4) although the previous
 // tile's xbar stores may be in flight too: vector-memory loads retire in
@@ -606,7 +631,7 @@ template <bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_bwd64d(const float* __restrict__ x, const float* __restrict__ ybar,
              float* __restrict__ xbar, const Geom g, const uint32_t n_orbits,
-             const float* __restrict__ ptm, const int64_t pstride, const GradOffs offs,
+             const float* __restrict__ ptm, const int64_t pstride, const BitOffs offs,
              double* __restrict__ partial, const BwdTiles tiles) {
   __shared__ __align__(16) char st0[2 * kDirArr];
   __shared__ __align__(16) char st1[2 * kDirArr];
@@ -620,15 +645,15 @@ __global__ void __launch_bounds__(kBlock)
   int64_t oin[2], oout[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    oin[h] = offs.off_in[8 * (2 * w + h) + e];
-    oout[h] = offs.off_out[8 * (2 * w + h) + e];
+    oin[h] = bit_off(offs.in, 8 * (2 * w + h) + e);
+    oout[h] = bit_off(offs.out, 8 * (2 * w + h) + e);
   }
   const uint32_t stride = tiles.stride;
   uint32_t t, ntiles;
   tiles.range(blockIdx.x, n_orbits / kDirTile, t, ntiles);
   if (t < ntiles) dir_issue<NT>(x, ybar, g, t, w, c, oin, oout, st0);
   const int n = lane & 15, kk = lane >> 4;
-  const int64_t xo = offs.off_in[16 * w + n];
+  const int64_t xo = bit_off(offs.in, 16 * w + n);
   float pb[16];
 #pragma unroll
   for (int s = 0; s < 16; ++s) pb[s] = ptm[(4 * s + kk) * 64 + 16 * w + n];
@@ -661,7 +686,7 @@ __global__ void __launch_bounds__(kBlock)
     }
     lds_barrier();
     dir_compute(st0, w, lane, acc);
-    bwd_apply(st0, pb, lane, g, t, xo, xbar);
+    dir_apply<false>(st0 + kDirArr, pb, lane, g, t, xo, xbar);
     if (++n_acc == kDirFlush) { flush(); n_acc = 0; }
     lds_barrier();
     if (t1 >= ntiles) break;
@@ -674,7 +699,7 @@ __global__ void __launch_bounds__(kBlock)
     }
     lds_barrier();
     dir_compute(st1, w, lane, acc);
-    bwd_apply(st1, pb, lane, g, t1, xo, xbar);
+    dir_apply<false>(st1 + kDirArr, pb, lane, g, t1, xo, xbar);
     if (++n_acc == kDirFlush) { flush(); n_acc = 0; }
     lds_barrier();
     t = t2;
@@ -810,7 +835,7 @@ template <bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_bwd64q(const float* __restrict__ x, const float* __restrict__ ybar,
              float* __restrict__ xbar, const Geom g, const uint32_t n_orbits,
-             const float* __restrict__ ptm, const int64_t pstride, const GradOffs offs,
+             const float* __restrict__ ptm, const int64_t pstride, const BitOffs offs,
              double* __restrict__ partial, const BwdTiles tiles) {
   __shared__ __align__(16) char st0[2 * kQArr];
   __shared__ __align__(16) char st1[2 * kQArr];
@@ -820,7 +845,7 @@ __global__ void __launch_bounds__(kBlock)
   ybar += int64_t(b) * g.bs_out;
   ptm += int64_t(b) * pstride;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int64_t oiq = offs.off_in[4 * (lane >> 2)], ooq = offs.off_out[4 * (lane >> 2)];
+  const int64_t oiq = bit_off(offs.in, 4 * (lane >> 2)), ooq = bit_off(offs.out, 4 * (lane >> 2));
   const uint32_t stride = tiles.stride;
   uint32_t t, ntiles;
   tiles.range(blockIdx.x, n_orbits / kDirTile, t, ntiles);
@@ -832,7 +857,7 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
   for (int sk = 0; sk < 16; ++sk)
     pa[sk] = ptm[(16 * (sk >> 2) + 4 * kk + (sk & 3)) * 64 + 16 * w + m];
-  const int64_t xo = offs.off_in[16 * w + 4 * kk];
+  const int64_t xo = bit_off(offs.in, 16 * w + 4 * kk);
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the PTM (and the first tile)
   typedef Mfma<float>::acc Acc;
   Acc acc[4];
@@ -936,7 +961,7 @@ template <bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_apply64q(const float* __restrict__ x, float* __restrict__ y, const Geom g,
                const uint32_t n_orbits, const float* __restrict__ ptm, const int64_t pstride,
-               const GradOffs offs) {
+               const BitOffs offs) {
   __shared__ __align__(16) char st0[kQArr];
   __shared__ __align__(16) char st1[kQArr];
   const uint32_t b = blockIdx.y;
@@ -944,13 +969,13 @@ __global__ void __launch_bounds__(kBlock)
   y += int64_t(b) * g.bs_out;
   ptm += int64_t(b) * pstride;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int64_t oiq = offs.off_in[4 * (lane >> 2)];
+  const int64_t oiq = bit_off(offs.in, 4 * (lane >> 2));
   const int m = lane & 15, kk = lane >> 4;
   float pa[16];
 #pragma unroll
   for (int sk = 0; sk < 16; ++sk)
     pa[sk] = ptm[(16 * w + m) * 64 + 16 * (sk >> 2) + 4 * kk + (sk & 3)];
-  const int64_t yo = offs.off_out[16 * w + 4 * kk];
+  const int64_t yo = bit_off(offs.out, 16 * w + 4 * kk);
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the PTM, before any tile load
   const uint32_t ntiles = n_orbits / kDirTile, stride = gridDim.x;
   uint32_t t = blockIdx.x;
@@ -981,7 +1006,6 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// Resident blocks of `kernel` over the device (occupancy x CUs).
 static uint32_t resident_blocks(const void* kernel) {
   int dev = 0, cus = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -993,6 +1017,61 @@ static uint32_t resident_blocks(const void* kernel) {
     per_cu = 1;
   (void)hipGetLastError();
   return uint32_t(per_cu) * uint32_t(cus);
+}
+
+// Float32 64 x 64 apply y = P x on orbit vectors of four (innermost axis a
+// bystander): x staged as k_bwd64d stages it (one operand), wave w computes
+// output entries 16w..16w+15 of the tile's 32 orbits (dir_apply with P's rows in
+// place of its columns): the k-steps of k_fused64<float, 1, 1, 4>, whose result it
+// has bit for bit.  That kernel stages the PTM in LDS, then a wave takes 64 orbits
+// and all 64 entries (256 MFMAs one after the other): right for bandwidth (its
+// loads in flight are four times these), too long a chain and too few blocks
+// where the states are small.  Here a block is one tile, its loads and the
+// PTM's under one latency, 32 MFMAs a wave.  Six states: 8 qubits 10.2 -> 3.9 us, 9
+// qubits 10.8 -> 6.4; two of 10 qubits 11.1 -> 7.6.  Used while all tiles are
+// resident at once: with more, k_fused64 is the faster (one of 11 qubits 11.6 us
+// against 15, six 45 against 51-57).
+template <bool NT>
+__device__ __forceinline__ void dir_issue_x(const float* x, const Geom& g, uint32_t t, int w,
+                                            int c, const int64_t (&oin)[2], char* lds) {
+  constexpr int kPol = NT ? 2 : 0;
+  int64_t bin, bout;
+  orbit_base(g, t * kDirTile + 4 * c, bin, bout);
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    __builtin_amdgcn_global_load_lds(x + bin + oin[h], lds + (2 * w + h) * kDirBlk, 16, 0, kPol);
+}
+
+template <bool NT>
+__global__ void __launch_bounds__(kBlock)
+    k_apply64d(const float* __restrict__ x, float* __restrict__ y, const Geom g,
+               const float* __restrict__ ptm, const int64_t pstride, const BitOffs offs) {
+  __shared__ __align__(16) char st[kDirArr];
+  const uint32_t b = blockIdx.y;
+  x += int64_t(b) * g.bs_in;
+  y += int64_t(b) * g.bs_out;
+  ptm += int64_t(b) * pstride;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int e = lane & 7, c = lane >> 3;
+  const int64_t oin[2] = {bit_off(offs.in, 16 * w + e), bit_off(offs.in, 16 * w + 8 + e)};
+  const uint32_t t = blockIdx.x;
+  dir_issue_x<NT>(x, g, t, w, c, oin, st);
+  const int n = lane & 15, kk = lane >> 4;
+  const int64_t yo = bit_off(offs.out, 16 * w + n);
+  float pb[16];
+  row_operand(ptm + (16 * w + n) * 64, kk, pb);
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+  lds_barrier();
+  dir_apply<true>(st, pb, lane, g, t, yo, y);
+}
+
+// Resident blocks of `kernel` over the device (occupancy x CUs).
+static uint32_t resident_blocks(const void* kernel);
+
+static uint32_t apply64d_cap() {
+  static const uint32_t cap =
+      resident_blocks(reinterpret_cast<const void*>(k_apply64d<true>));
+  return cap;
 }
 
 // Host side of k_apply64q: natural per-entry offsets from the fused plan's
@@ -1014,12 +1093,37 @@ int launch_apply64q(const FusedPlan& fp, const Geom& g, bool nt, const void* in,
   static const uint32_t cap =
       resident_blocks(reinterpret_cast<const void*>(k_apply64q<true>));
   const uint32_t tiles = fp.n_orbits / kDirTile;
-  uint32_t nb = cap / std::max<uint32_t>(batch, 1);
-  nb = std::max<uint32_t>(1, std::min(nb, std::max<uint32_t>(tiles / 4, 1)));
+  // one round of resident blocks over the batch: a tile each where that holds
+  // them all (six states of 8 qubits 6.6 -> 3.7 us, of 9 qubits 7.5 -> 6.0), else at
+  // least four
+  batch = std::max<uint32_t>(batch, 1);
+  uint32_t nb = tiles;
+  if (uint64_t(tiles) * batch > cap) nb = std::min(cap / batch, tiles / 4);
+  nb = std::max<uint32_t>(1, nb);
   auto kern = nt ? k_apply64q<true> : k_apply64q<false>;
   hipLaunchKernelGGL(kern, dim3(nb, batch), dim3(kBlock), 0, s, static_cast<const float*>(in),
                      static_cast<float*>(out), g, fp.n_orbits,
-                     static_cast<const float*>(ptm_rows), pstride, o);
+                     static_cast<const float*>(ptm_rows), pstride, bit_offs(o));
+  QSV_CHECK_HIP(hipGetLastError());
+  return QSV_OK;
+}
+
+bool apply64d_applies(int elem_bytes, const FusedPlan& fp, uint32_t batch) {
+  return elem_bytes == 4 && fp.D == 64 && fp.vn == 4 && fp.n_orbits % kDirTile == 0 &&
+         uint64_t(fp.n_orbits / kDirTile) * batch <= apply64d_cap();
+}
+
+int launch_apply64d(const FusedPlan& fp, const Geom& g, bool nt, const void* in, void* out,
+                    const void* ptm_rows, int64_t pstride, uint32_t batch, hipStream_t s) {
+  GradOffs o;
+  for (int q = 0; q < 16; ++q)
+    for (int j = 0; j < 4; ++j) {
+      o.off_in[4 * q + j] = fp.offs.in_u[q] + fp.offs.in_l[j];
+      o.off_out[4 * q + j] = fp.offs.out_u[q] + fp.offs.out_l[j];
+    }
+  auto kern = nt ? k_apply64d<true> : k_apply64d<false>;
+  hipLaunchKernelGGL(kern, dim3(fp.n_orbits / kDirTile, batch), dim3(kBlock), 0, s, static_cast<const float*>(in),
+                     static_cast<float*>(out), g, static_cast<const float*>(ptm_rows), pstride, bit_offs(o));
   QSV_CHECK_HIP(hipGetLastError());
   return QSV_OK;
 }
@@ -2499,8 +2603,8 @@ static int batched_backward_run(int dtype, const void* x, const void* ybar, void
                        : (nt ? k_bwd64d<true> : k_bwd64d<false>);
     hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, s, static_cast<const float*>(x),
                        static_cast<const float*>(ybar), static_cast<float*>(xbar), p.g,
-                       p.n_orbits, static_cast<const float*>(ptm_dev), ptm_batch_stride, p.offs,
-                       partial, tiles);
+                       p.n_orbits, static_cast<const float*>(ptm_dev), ptm_batch_stride,
+                       bit_offs(p.offs), partial, tiles);
   } else
     hipLaunchKernelGGL((k_bwd64<double, 2>), grid, dim3(kBlock), 0, s,
                        static_cast<const double*>(x), static_cast<const double*>(ybar),
@@ -2763,9 +2867,9 @@ static int emulate_apply64q(const GradPlan& p, const double* x, const double* pt
   return QSV_OK;
 }
 
-extern "C" int qsv_emulate_apply_ptm_direct(int dtype, const double* x, double* y, int rank,
-                                            const int64_t* dims, int k, const int32_t* targets,
-                                            const double* ptm, int32_t blocks) {
+static int emulate_apply_direct(bool quad, int dtype, const double* x, double* y, int rank,
+                                const int64_t* dims, int k, const int32_t* targets,
+                                const double* ptm, int32_t blocks) {
   QSV_CHECK_ARG(dtype == QSV_F32 || dtype == QSV_F64, "unknown dtype %d", dtype);
   QSV_CHECK_ARG(dims && targets && k >= 1 && k <= QSV_MAX_TARGETS && rank >= 1 &&
                     rank <= QSV_MAX_RANK,
@@ -2778,9 +2882,10 @@ extern "C" int qsv_emulate_apply_ptm_direct(int dtype, const double* x, double* 
   GradPlan p;
   const int rc = make_grad_plan(dtype_size(dtype), rank, dims, k, targets, dout, p);
   if (rc) return rc;
-  if (dtype != QSV_F32 || !bwd64q_applies(p)) {
-    set_error("the direct 64 x 64 apply takes float32 states whose PTM's lowest index is the "
-              "innermost axis, on whole %d-orbit tiles", kDirTile);
+  if (dtype != QSV_F32 ||
+      !(quad ? bwd64q_applies(p) : bwd64_applies(p) && grad64_direct(p, 4, p.vn))) {
+    set_error("the direct 64 x 64 apply takes float32 states whose %s, on whole %d-orbit tiles",
+              quad ? "PTM's lowest index is the innermost axis" : "orbits come in fours", kDirTile);
     return QSV_ENOTSUP;
   }
   QSV_CHECK_ARG(x && y && ptm, "null pointer argument");
@@ -2788,7 +2893,25 @@ extern "C" int qsv_emulate_apply_ptm_direct(int dtype, const double* x, double* 
   QSV_CHECK_ARG(blocks >= 0 && blocks <= 4096, "blocks outside [0, 4096]");
   const uint32_t tiles = p.n_orbits / kDirTile;
   const int nb = blocks > 0 ? blocks : int(std::max<uint32_t>(1, tiles / 4));
-  return emulate_apply64q(p, x, ptm, nb, y);
+  if (quad) return emulate_apply64q(p, x, ptm, nb, y);
+  // k_apply64d is k_bwd64d's staging of ybar and its apply half, here of x with
+  // the transposed PTM (input and output are laid out alike)
+  std::vector<double> pt(64 * 64), dp(64 * 64);
+  for (int o = 0; o < 64; ++o)
+    for (int i = 0; i < 64; ++i) pt[i * 64 + o] = ptm[o * 64 + i];
+  return emulate_grad64d(p, x, x, {uint32_t(nb), 1, 0}, dp.data(), pt.data(), y);
+}
+
+extern "C" int qsv_emulate_apply_ptm_direct(int dtype, const double* x, double* y, int rank,
+                                            const int64_t* dims, int k, const int32_t* targets,
+                                            const double* ptm, int32_t blocks) {
+  return emulate_apply_direct(true, dtype, x, y, rank, dims, k, targets, ptm, blocks);
+}
+
+extern "C" int qsv_emulate_apply_ptm_vectors(int dtype, const double* x, double* y, int rank,
+                                             const int64_t* dims, int k, const int32_t* targets,
+                                             const double* ptm, int32_t blocks) {
+  return emulate_apply_direct(false, dtype, x, y, rank, dims, k, targets, ptm, blocks);
 }
 
 // Host replay of k_bwd64 + k_ptm_grad_final for one state.  Part A: every
