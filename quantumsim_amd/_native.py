@@ -66,7 +66,7 @@ _SIGNATURES = {
                                      ctypes.c_int64, _vp]),
     'qsv_apply_ptm_strided': (ctypes.c_int, [ctypes.c_int, _vp, _vp, ctypes.c_int, _c_i64p,
                                              _c_i64p, _c_i64p, ctypes.c_int, _c_i32p, _c_i32p,
-                                             _c_f64p, _vp, ctypes.c_int64, _vp]),
+                                             _vp, _vp, ctypes.c_int64, _vp]),
     'qsv_apply_ptm_dev': (ctypes.c_int, [ctypes.c_int, _vp, _vp, ctypes.c_int, _c_i64p,
                                          ctypes.c_int, _c_i32p, _c_i32p, _vp, _vp,
                                          ctypes.c_int64, _vp]),

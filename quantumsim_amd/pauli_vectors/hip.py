@@ -8,6 +8,7 @@ request); every operation on it runs in libqsv's HIP kernels, launched on
 torch's current stream.  Readouts (diagonal, trace, meas_prob) are computed
 and returned in float64 whatever the state's element type.
 """
+import functools
 import math
 import os
 import warnings
@@ -52,8 +53,26 @@ def _resolve_device(device):
     return device
 
 
+def _raw_stream(device):
+    """Handle of torch's current stream (0: the default stream); without the
+    stream object, which costs a tenth of a small vector's gate to build."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
 def _stream(device):
-    return ctypes_void(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes_void(_raw_stream(device))
+
+
+@functools.lru_cache(maxsize=4096)
+def _i32s(values):
+    """A tuple as the library's int32 array (read-only there)."""
+    return nat.i32(values)
+
+
+@functools.lru_cache(maxsize=1024)
+def _ptm_workspace(code, dims_in, dims_out):
+    return nat.check(nat.lib().qsv_apply_ptm_workspace_bytes(
+        code, len(dims_in), _i32s(dims_in), _i32s(dims_out)), 'apply_ptm')
 
 
 def ctypes_void(v):
@@ -73,7 +92,7 @@ class _Scratch:
 
     @classmethod
     def get(cls, device, purpose, nbytes):
-        key = (device, torch.cuda.current_stream(device).cuda_stream, purpose)
+        key = (device, _raw_stream(device), purpose)
         t = cls._bufs.get(key)
         if t is None or t.numel() < nbytes:
             t = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -196,8 +215,10 @@ class PauliVectorHIP(PauliVectorBase):
             view.copy_(pv.detach().to(device=self._device, dtype=self._dtype))
         else:
             view[(0,) * len(self._shape)] = 1
+        store._qsv_home = _raw_stream(self._device)
         self._store = store           # owning storage of the state
         self._data = store            # physical (padded) extent
+        self._geo = (None, None, None, None)
         self._spare = None            # second buffer (apply_ptm writes there)
 
     # ------------------------------------------------------------ plumbing
@@ -232,25 +253,35 @@ class PauliVectorHIP(PauliVectorBase):
         go back to that stream's pool when it is dropped (a spare replaced by
         a larger one, the vector deleted) and could be handed out again while
         this stream's kernels still read or write it; the caching allocator
-        ignores the mark for a buffer's own allocation stream."""
-        cur = torch.cuda.current_stream(self._device)
+        ignores the mark for a buffer's own allocation stream, so buffers
+        known to be this stream's (_qsv_home) are not marked."""
+        raw = _raw_stream(self._device)
         for t in tensors:
-            if t is not None:
-                t.record_stream(cur)
+            if t is not None and getattr(t, '_qsv_home', None) != raw:
+                t.record_stream(torch.cuda.current_stream(self._device))
 
     def _take_spare(self, n):
         sp = self._spare
         if sp is None or sp.numel() < n:
             sp = torch.empty(max(n, 1), dtype=self._dtype, device=self._device)
+            sp._qsv_home = _raw_stream(self._device)
         self._spare = None
         return sp
 
     def _swap_in(self, store, extent, shape, strides):
         self._spare = self._store
         self._store = store
-        self._data = store[:extent]
+        self._data = store if store.numel() == extent else store[:extent]
         self._shape = tuple(shape)
         self._pstr = tuple(strides)
+
+    def _geometry(self):
+        """The layout's dims and strides as the library's arrays."""
+        geo = self._geo
+        if geo[0] is not self._shape or geo[1] is not self._pstr:
+            geo = self._geo = (self._shape, self._pstr, nat.i64(self._shape),
+                               nat.i64(self._pstr))
+        return geo[2], geo[3]
 
     # ----------------------------------------------------------------- API
     def to_pv(self):
@@ -262,21 +293,22 @@ class PauliVectorHIP(PauliVectorBase):
         the caller updates it (quantumsim/operations/operation.py:549-551)."""
         # a PTM already on this vector's device stays there (no host copy,
         # no synchronisation): the device-side operation pipeline
-        on_device = (isinstance(ptm, torch.Tensor) and ptm.device.type == 'cuda'
-                     and ptm.device == self._device)
-        if isinstance(ptm, torch.Tensor) and not on_device:
-            ptm = ptm.detach().cpu().numpy()
+        on_device = False
+        if isinstance(ptm, torch.Tensor):
+            on_device = ptm.device.type == 'cuda' and ptm.device == self._device
+            if not on_device:
+                ptm = ptm.detach().cpu().numpy()
         if not on_device:
             ptm = np.asarray(ptm)
         k = len(qubits)
         if ptm.ndim != 2 * k:
             raise ValueError('{}-qubit PTM must have {} dimensions, got {}'
                              .format(k, 2 * k, ptm.ndim))
-        if (ptm.is_complex() if on_device else np.iscomplexobj(ptm)):
+        if (ptm.is_complex() if on_device else ptm.dtype.kind == 'c'):
             raise ValueError('PTM must be real, got dtype {}'.format(ptm.dtype))
         if k == 0:
             raise ValueError('apply_ptm needs at least one qubit')
-        qubits = tuple(int(q) for q in qubits)
+        qubits = tuple([int(q) for q in qubits])
         for q in qubits:
             self._validate_qubit(q, 'qubit')
         if len(set(qubits)) != k:
@@ -284,13 +316,14 @@ class PauliVectorHIP(PauliVectorBase):
         if k > 8:
             raise NotImplementedError('Applying {}-qubit PTM is not implemented in the '
                                       'active backend.'.format(k))
-        dims_out_t = ptm.shape[:k]
-        dims_in_t = ptm.shape[k:]
+        dims = tuple(ptm.shape)
+        dims_out_t, dims_in_t = dims[:k], dims[k:]
+        shape = self._shape
         for q, d in zip(qubits, dims_in_t):
-            if self._shape[q] != d:
+            if shape[q] != d:
                 raise ValueError('PTM input dimension {} does not match dimension {} of '
-                                 'qubit {}'.format(d, self._shape[q], q))
-        if not on_device and math.prod(dims_in_t) in (64, 256) and dims_in_t == dims_out_t:
+                                 'qubit {}'.format(d, shape[q], q))
+        if not on_device and dims_in_t == dims_out_t and math.prod(dims_in_t) in (64, 256):
             # dense 3-/4-qubit PTMs from the host: staged through pinned
             # memory and copied asynchronously, then applied as a device PTM
             # (the MFMA kernels gather or pack it on the device), so the call
@@ -303,31 +336,27 @@ class PauliVectorHIP(PauliVectorBase):
             on_device = True
         if on_device:
             ptm = ptm.detach().to(self._dtype).contiguous()
-        else:
+        elif ptm.dtype != np.float64 or not ptm.flags.c_contiguous:
             ptm = np.ascontiguousarray(ptm, dtype=np.float64)
-        new_shape = list(self._shape)
-        for q, d in zip(qubits, dims_out_t):
-            new_shape[q] = d
-        new_str, extent = physical_strides(new_shape, self._elem_bytes())
+        in_dims, in_str = self._geometry()
+        if dims_out_t == dims_in_t:              # the layout stays
+            new_shape, new_str, extent, out_str = shape, self._pstr, self._data.numel(), in_str
+        else:
+            new_shape = list(shape)
+            for q, d in zip(qubits, dims_out_t):
+                new_shape[q] = d
+            new_str, extent = physical_strides(new_shape, self._elem_bytes())
+            out_str = nat.i64(new_str)
         out = self._take_spare(extent)
         code = self._code()
-        L = nat.lib()
-        ws_bytes = L.qsv_apply_ptm_workspace_bytes(code, k, nat.i32(dims_in_t),
-                                                   nat.i32(dims_out_t))
-        nat.check(ws_bytes, 'apply_ptm')
+        ws_bytes = _ptm_workspace(code, dims_in_t, dims_out_t)
         ws = _Scratch.get(self._device, 'ptm', ws_bytes).data_ptr() if ws_bytes else None
-        if on_device:
-            rc = L.qsv_apply_ptm_dev_strided(
-                code, self._store.data_ptr(), out.data_ptr(), len(self._shape),
-                nat.i64(self._shape), nat.i64(self._pstr), nat.i64(new_str), k,
-                nat.i32(qubits), nat.i32(dims_out_t), ptm.data_ptr(), ws, ws_bytes,
-                _stream(self._device))
-        else:
-            rc = L.qsv_apply_ptm_strided(
-                code, self._store.data_ptr(), out.data_ptr(), len(self._shape),
-                nat.i64(self._shape), nat.i64(self._pstr), nat.i64(new_str), k,
-                nat.i32(qubits), nat.i32(dims_out_t), ptm.ctypes.data_as(nat._c_f64p), ws,
-                ws_bytes, _stream(self._device))
+        L = nat.lib()
+        apply, data = ((L.qsv_apply_ptm_dev_strided, ptm.data_ptr()) if on_device else
+                       (L.qsv_apply_ptm_strided, ptm.__array_interface__['data'][0]))
+        rc = apply(code, self._store.data_ptr(), out.data_ptr(), len(shape), in_dims, in_str,
+                   out_str, k, _i32s(qubits), _i32s(dims_out_t), data, ws, ws_bytes,
+                   _stream(self._device))
         if rc != 0:
             self._spare = out
             nat.check(rc, 'apply_ptm')
