@@ -94,24 +94,22 @@ __global__ void __launch_bounds__(kBlock)
   in += int64_t(blockIdx.y) * g.bs_in;
   out += int64_t(blockIdx.y) * g.bs_out;
   pf += int64_t(blockIdx.y) * pstride;
-  if (prow && sizeof(T) == 4) {
+  if (prow) {
     // wave w makes the fragments of row block w, a row per lane (row_operand,
     // runs of four as they are): gathered one by one, each load touched sixteen
-    // cache lines (six states of 10 qubits 19.0 -> 16.8 us, of 11 qubits 49 -> 45)
+    // cache lines (six float32 states of 10 qubits 19.0 -> 16.8 us, of 11 qubits
+    // 49 -> 45; float64, two of 10 qubits 13.4 -> 11.9, one of 11 21.5 -> 18.5)
     const int ln = threadIdx.x & 63, w = threadIdx.x >> 6, jj = ln >> 4;
-    const T* row = pf + fused_frag_source(64, 4, VI, VO, w * 64 + (ln & 15));
-    float v[KS];
+    const T* row = pf + fused_frag_source(64, int(sizeof(T)), VI, VO, w * 64 + (ln & 15));
+    T v[KS];
     if constexpr (VI == 1) {
-      row_operand(reinterpret_cast<const float*>(row), jj, v);
+      row_operand(row, jj, v);
     } else {
 #pragma unroll
-      for (int s = 0; s < KS; ++s) v[s] = row[16 * (s >> 2) + 4 * jj + (s & 3)];
+      for (int s = 0; s < KS; ++s) v[s] = row[fused_k(VI, s, jj)];
     }
 #pragma unroll
     for (int s = 0; s < KS; ++s) As[(s * MB + w) * 64 + ln] = v[s];
-  } else if (prow) {
-    for (int i = threadIdx.x; i < KS * MB * 64; i += kBlock)
-      As[i] = pf[fused_frag_source(64, int(sizeof(T)), VI, VO, i)];
   } else {
     for (int i = threadIdx.x; i < KS * MB * 64; i += kBlock) As[i] = pf[i];
   }
