@@ -354,7 +354,8 @@ class _SchedulePositions:
             if tile is not None:
                 r.apply = tile
             if self.grads is not None and self.grads[p] is not None:
-                tile = tuner.grad_tile(dtype, active, self.shape, tg, d)
+                # (the one-pass backward takes no launch shape)
+                tile = None if r.fused else tuner.grad_tile(dtype, active, self.shape, tg, d)
                 r.has_grad = tile is not None
                 if tile is not None:
                     r.grad = tile
