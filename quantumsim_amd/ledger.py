@@ -38,7 +38,7 @@ PERSISTENT_ADJ = 'persistent_adjoint'
 
 # the HIP kernels behind each family (rocprofv3 names)
 KERNELS = {
-    APPLY_DENSE64: 'k_fused64 / k_apply64q (64 x 64 PTMs on MFMA)',
+    APPLY_DENSE64: 'k_fused64 / k_apply64q / k_apply64d (64 x 64 PTMs on MFMA)',
     APPLY_SMALL: 'k_apply_small / k_apply_lds (PTMs up to 16 x 16)',
     GRAD_DENSE64: 'k_ptm_grad64 / k_ptm_grad64d + k_ptm_grad_final',
     GRAD_SMALL: 'k_ptm_grad + k_ptm_grad_final',
