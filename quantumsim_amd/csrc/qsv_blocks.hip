@@ -380,11 +380,16 @@ __host__ __device__ __forceinline__ void wb_load(int tid, int nthr, const qsv_wb
 }
 
 // ------------------------------------------------------------ kernels
-template <typename T>
+// ONE: every position is one factor on one or two qubits (a circuit's gates by
+// themselves): 6 KB of LDS instead of 48, so eight workgroups a CU instead of
+// three (the gates of 192 circuits of 4-7 qubits 346 -> 196 us).  The backward gains
+// nothing from the same (594 us, 628 with 14.5 KB) and has one form.
+template <typename T, bool ONE>
 __global__ void __launch_bounds__(kWB)
     k_window_blocks(const qsv_wblock* __restrict__ table, const WBGeom g, T* __restrict__ out,
                     int64_t out_elems) {
-  __shared__ double F[4 * 256], Tm[4 * 256], M[64 * 64];
+  constexpr int NF = ONE ? 1 : 4, MD = ONE ? 16 : 64;
+  __shared__ double F[NF * 256], Tm[NF * 256], M[MD * MD];
   const int b = blockIdx.x, w = blockIdx.y;
   const qsv_wblock& blk = table[blockIdx.z];  // uniform: scalar loads, no private copy
   const int tid = threadIdx.x;
@@ -504,16 +509,25 @@ static int wb_geom(int batch, int n_windows, int span, int n_qubits, int layers,
   return QSV_OK;
 }
 
-static int wb_run(int dtype, int n_pos, const qsv_wblock* table_dev, const WBGeom& g, void* out,
-                  int64_t out_elems, void* stream) {
+// Every position one factor on at most two qubits (kernels with ONE).
+static bool wb_one(int n_pos, const qsv_wblock* table) {
+  for (int p = 0; p < n_pos; ++p)
+    if (table[p].nf != 1 || table[p].nq > 2) return false;
+  return true;
+}
+
+static int wb_run(int dtype, int n_pos, const qsv_wblock* table_host,
+                  const qsv_wblock* table_dev, const WBGeom& g, void* out, int64_t out_elems,
+                  void* stream) {
   QSV_CHECK_ARG(table_dev && out, "null pointer argument");
   const dim3 grid(g.batch, g.nw, n_pos);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool one = wb_one(n_pos, table_host);
   if (dtype == QSV_F64)
-    hipLaunchKernelGGL(k_window_blocks<double>, grid, dim3(kWB), 0, s, table_dev, g,
+    hipLaunchKernelGGL((one ? k_window_blocks<double, true> : k_window_blocks<double, false>), grid, dim3(kWB), 0, s, table_dev, g,
                        static_cast<double*>(out), out_elems);
   else
-    hipLaunchKernelGGL(k_window_blocks<float>, grid, dim3(kWB), 0, s, table_dev, g,
+    hipLaunchKernelGGL((one ? k_window_blocks<float, true> : k_window_blocks<float, false>), grid, dim3(kWB), 0, s, table_dev, g,
                        static_cast<float*>(out), out_elems);
   QSV_CHECK_HIP(hipGetLastError());
   return QSV_OK;
@@ -547,7 +561,7 @@ extern "C" int qsv_window_blocks(int dtype, int n_pos, const qsv_wblock* table_h
   if (rc) return rc;
   rc = check_table(table_host, n_pos, n_qubits, out_elems, batch, n_windows, 2, 64);
   if (rc) return rc;
-  return wb_run(dtype, n_pos, table_dev, g, out, out_elems, stream);
+  return wb_run(dtype, n_pos, table_host, table_dev, g, out, out_elems, stream);
 }
 
 extern "C" int qsv_window_blocks_backward(int dtype, int n_pos, const qsv_wblock* table_host,
@@ -576,7 +590,7 @@ extern "C" int qsv_layer_blocks(int dtype, int n_pos, const qsv_wblock* table_ho
   if (rc) return rc;
   rc = check_table(table_host, n_pos, n_qubits, out_elems, batch, 1, layers, 65535);
   if (rc) return rc;
-  return wb_run(dtype, n_pos, table_dev, g, out, out_elems, stream);
+  return wb_run(dtype, n_pos, table_host, table_dev, g, out, out_elems, stream);
 }
 
 extern "C" int qsv_layer_blocks_backward(int dtype, int n_pos, const qsv_wblock* table_host,
