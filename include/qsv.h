@@ -290,6 +290,12 @@ int qsv_emulate_window_blocks(int n_pos, const qsv_wblock* table, int batch, int
                               int64_t out_elems, const double* dout, double* drot,
                               double* ddamp_part);
 
+/* Writes `bytes` (a multiple of 4, at most 16 MB) of host memory to device
+ * memory on `stream`, inside the launches' arguments (3.5 KB each): for tables of
+ * a few KB.  The source may change once the call has returned, and a HIP graph
+ * that captures the call keeps the bytes themselves. */
+int qsv_put(const void* host, int64_t bytes, void* dst, void* stream);
+
 /* The same blocks for one window over all `layers` layers (f_layer in
  * [0, layers)): the blocks of any fusion plan of the layered circuit, each
  * gate in one block; ddamp_part is [batch][layers][n_qubits][4][4]. */

@@ -128,6 +128,7 @@ _SIGNATURES = {
                                  [ctypes.c_double] + [_vp] * 4),
     'qsv_emulate_gate_params': (ctypes.c_int, [ctypes.c_int] * 4 + [_vp] * 5 + [ctypes.c_double] +
                                 [_vp] * 6),
+    'qsv_put': (ctypes.c_int, [_vp, ctypes.c_int64, _vp, _vp]),
     'qsv_layer_blocks': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _vp, _vp, ctypes.c_int,
                                         ctypes.c_int, ctypes.c_int, _vp, _vp, _vp, _vp,
                                         ctypes.c_int64, _vp]),

@@ -27,6 +27,7 @@
 #include "qsv_common.h"
 
 #include <string.h>
+#include <algorithm>
 #include <vector>
 
 namespace qsv {
@@ -458,6 +459,17 @@ __global__ void __launch_bounds__(kWB)
   }
 }
 
+// A few KB of host memory to the device by value, in the launch's arguments: the
+// source is free once the call returns, and a captured launch keeps its own copy.
+constexpr int kPutWords = 896;  // 3.5 KB of the 4 KB of arguments
+struct PutChunk {
+  uint32_t w[kPutWords];
+};
+__global__ void __launch_bounds__(kWB) k_put(const PutChunk c, uint32_t* __restrict__ dst, int n) {
+  const int i = blockIdx.x * kWB + threadIdx.x;
+  if (i < n) dst[i] = c.w[i];
+}
+
 // ------------------------------------------------------------ host side
 static int check_table(const qsv_wblock* t, int npos, int n, int64_t out_elems, int batch,
                        int nw, int span, int most) {
@@ -546,6 +558,23 @@ static int wb_run_backward(int dtype, int n_pos, const qsv_wblock* table_dev, co
     hipLaunchKernelGGL(k_window_blocks_bwd<float>, grid, dim3(kWB), 0, s, table_dev, g,
                        static_cast<const float*>(dout), out_elems, drot, ddamp_part);
   QSV_CHECK_HIP(hipGetLastError());
+  return QSV_OK;
+}
+
+extern "C" int qsv_put(const void* host, int64_t bytes, void* dst, void* stream) {
+  QSV_CHECK_ARG(bytes >= 0 && bytes % 4 == 0 && bytes <= (int64_t(1) << 24),
+                "%lld bytes to put: a multiple of 4, at most 16 MB", (long long)bytes);
+  if (bytes == 0) return QSV_OK;
+  QSV_CHECK_ARG(host && dst && reinterpret_cast<uintptr_t>(dst) % 4 == 0, "bad pointer argument");
+  for (int64_t at = 0; at < bytes; at += int64_t(kPutWords) * 4) {
+    const int n = int(std::min<int64_t>(bytes - at, int64_t(kPutWords) * 4) / 4);
+    PutChunk c;
+    memcpy(c.w, static_cast<const char*>(host) + at, size_t(n) * 4);
+    hipLaunchKernelGGL(k_put, dim3((n + kWB - 1) / kWB), dim3(kWB), 0,
+                       static_cast<hipStream_t>(stream), c, static_cast<uint32_t*>(dst) + at / 4,
+                       n);
+    QSV_CHECK_HIP(hipGetLastError());
+  }
   return QSV_OK;
 }
 

@@ -54,6 +54,14 @@ def _to_device(table, device):
     return None if device is None else torch.from_numpy(table.view(np.uint8).copy()).to(device)
 
 
+def _put(host, device):
+    """A numpy array's bytes on ``device``, written by launches that carry them
+    (qsv_put): a captured graph needs neither the array nor this tensor after."""
+    out = torch.empty(host.nbytes, dtype=torch.uint8, device=device)
+    nat.check(nat.lib().qsv_put(host.ctypes.data, host.nbytes, out.data_ptr(), _stream()), 'put')
+    return out
+
+
 class WindowPlan:
     """The block table of an n-qubit group with ``n_windows`` windows and
     ``batch`` circuits: per block position its qubits, factors (a lone qubit
@@ -107,7 +115,10 @@ class LayerBlockPlan:
     qubits (fusion.fuse_plan of its gates, blocks of up to three qubits) for
     ``batch`` parameter sets.  A block of more than four gates is built as
     two, in the last positions, and multiplied (``split``: block index ->
-    (offset of the first part, of the second))."""
+    (offset of the first part, of the second)).  Host memory only:
+    layer_blocks writes the table to the device in every call, so that a
+    captured step depends on no plan's lifetime.  ``device``: the only one the
+    plan is used on (None: any)."""
 
     def __init__(self, n, layers, batch, device=None):
         self.n, self.layers, self.batch = n, layers, batch
@@ -141,7 +152,6 @@ class LayerBlockPlan:
         self.split_D = self.blocks[split[0]][1] if split else 0
         self.out_elems = off
         self.device = device
-        self.table_dev = _to_device(self.table, device)
 
     def host_ptr(self):
         return self.table.ctypes.data_as(nat.ctypes.c_void_p)
@@ -215,12 +225,16 @@ class _LayerBlocks(torch.autograd.Function):
     def forward(ctx, rot, damp, which, plan, dtype, cz):
         # every layer's own rotations: the factors' gradients have one writer
         # per (layer, qubit)
-        full = rot.detach().index_select(1, which) if which is not None else rot.detach()
+        full, index = rot.detach(), None
+        if which is not None:
+            index = _put(np.array(which, dtype=np.int64), rot.device).view(torch.int64)
+            full = full.index_select(1, index)
         full = full.contiguous()
         damp = damp.detach().contiguous()
+        table = _put(plan.table, rot.device)
         out = torch.empty(plan.out_elems, dtype=torch.float64, device=rot.device)
         rc = nat.lib().qsv_layer_blocks(
-            nat.QSV_F64, len(plan.table), plan.host_ptr(), plan.table_dev.data_ptr(), plan.batch,
+            nat.QSV_F64, len(plan.table), plan.host_ptr(), table.data_ptr(), plan.batch,
             plan.n, plan.layers, full.data_ptr(), damp.data_ptr(), cz.data_ptr(), out.data_ptr(),
             plan.out_elems, _stream())
         nat.check(rc, 'layer_blocks')
@@ -232,8 +246,8 @@ class _LayerBlocks(torch.autograd.Function):
             prod = torch.bmm(second, first).to(dtype)
         whole = out[:plan.whole_elems].to(dtype)
         ctx.plan, ctx.dtype, ctx.n_rot = plan, dtype, rot.shape[1]
-        saved = [full, damp, cz] + ([first, second] if S else []) + \
-                ([which] if which is not None else [])
+        saved = [full, damp, cz, table] + ([first, second] if S else []) + \
+                ([index] if index is not None else [])
         ctx.parts = (bool(S), which is not None)
         ctx.save_for_backward(*saved)
         res = []
@@ -250,7 +264,7 @@ class _LayerBlocks(torch.autograd.Function):
     def backward(ctx, *grads):
         plan = ctx.plan
         saved = list(ctx.saved_tensors)
-        full, damp, cz = saved[:3]
+        full, damp, cz, table = saved[:4]
         has_split, has_which = ctx.parts
 
         def flat(k):
@@ -261,7 +275,7 @@ class _LayerBlocks(torch.autograd.Function):
         # dict order is the table's: whole blocks by offset
         parts = [torch.cat([flat(k) for k in plan.offset]).double()] if plan.offset else []
         if has_split:
-            first, second = saved[3:5]
+            first, second = saved[4:6]
             g = torch.cat([flat(k) for k in plan.split]).double().view_as(first)
             parts.append(torch.bmm(second.transpose(1, 2).contiguous(), g).reshape(-1))
             parts.append(torch.bmm(g, first.transpose(1, 2).contiguous()).reshape(-1))
@@ -270,7 +284,7 @@ class _LayerBlocks(torch.autograd.Function):
         ddp = torch.empty((plan.batch, plan.layers, plan.n, 4, 4), dtype=torch.float64,
                           device=full.device)
         rc = nat.lib().qsv_layer_blocks_backward(
-            nat.QSV_F64, len(plan.table), plan.host_ptr(), plan.table_dev.data_ptr(), plan.batch,
+            nat.QSV_F64, len(plan.table), plan.host_ptr(), table.data_ptr(), plan.batch,
             plan.n, plan.layers, full.data_ptr(), damp.data_ptr(), cz.data_ptr(), dout.data_ptr(),
             plan.out_elems, dfull.data_ptr(), ddp.data_ptr(), _stream())
         nat.check(rc, 'layer_blocks_backward')
@@ -291,7 +305,8 @@ def layer_blocks(rot, damp, plan, dtype, cz, which=None):
     respect to ``rot`` [batch, sets, n, 4, 4] (layer l uses set which[l]; None:
     one set per layer) and ``damp`` [batch, n, 4, 4], both float64.  The values
     of fusion.fuse_batched over workloads.fused_layer_gates, in two launches
-    (one forward, one backward) and two small products."""
+    (one forward, one backward), the table's few and two small products.
+    ``which``: host integers (a device tensor is read back first)."""
     sets = rot.shape[1]
     n_sets = plan.layers if which is None else sets
     if tuple(rot.shape) != (plan.batch, n_sets, plan.n, 4, 4) or \
@@ -300,8 +315,12 @@ def layer_blocks(rot, damp, plan, dtype, cz, which=None):
                          '%d qubits' % (tuple(rot.shape), tuple(damp.shape), plan.batch, plan.n))
     if rot.dtype != torch.float64 or damp.dtype != torch.float64:
         raise ValueError('rotation and damping PTMs must be float64')
-    if which is not None and (which.dtype != torch.int64 or tuple(which.shape) != (plan.layers,)):
-        raise ValueError('which must hold one rotation set per layer')
+    if which is not None:
+        which = tuple(int(w) for w in (which.tolist() if hasattr(which, 'tolist') else which))
+        if len(which) != plan.layers:
+            raise ValueError('which must hold one rotation set per layer')
+    if plan.device is not None and torch.device(plan.device).type != rot.device.type:
+        raise ValueError('a plan for %s, rotation PTMs on %s' % (plan.device, rot.device))
     out = _LayerBlocks.apply(rot, damp, which, plan, dtype, cz)
     return [(m, qs) for m, (qs, _) in zip(out, plan.blocks)]
 

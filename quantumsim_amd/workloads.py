@@ -331,6 +331,13 @@ def _gate_ptms_function():
     return GatePTMs
 
 
+@functools.lru_cache(maxsize=32)
+def _layer_plan(n, layers, sets):
+    """windows.LayerBlockPlan, kept for the circuits last used (host memory)."""
+    from .windows import LayerBlockPlan
+    return LayerBlockPlan(n, layers, sets)
+
+
 class TrainableCircuit:
     """12 qubits, 40 layers, 96 trainable parameters per parameter set:
     RX/RZ angles shared by the layers of a 5-layer block, three blocks used
@@ -344,7 +351,6 @@ class TrainableCircuit:
     def __init__(self, n=12, layers=40, block=5, n_blocks=3):
         self.n, self.layers, self.block, self.n_blocks = n, layers, block, n_blocks
         self.n_params = n_blocks * n * 2 + 2 * n
-        self._plans = {}           # block plans per (sets, device)
 
     def initial_params(self, sets, seed, device, dtype):
         import torch
@@ -372,21 +378,10 @@ class TrainableCircuit:
         return out
 
     def _blocks(self, ang, t1, t2, dtype):
-        import torch
-        from .autograd import Gate, cz_ptm, shared_constant
-        from .windows import LayerBlockPlan, layer_blocks
-        key = (ang.shape[0], ang.device)
-        hit = self._plans.get(key)
-        if hit is None:
-            plan = LayerBlockPlan(self.n, self.layers, ang.shape[0], ang.device)
-            which = torch.tensor([(layer // self.block) % self.n_blocks
-                                  for layer in range(self.layers)], device=ang.device)
-            shared_constant(plan.table_dev)
-            hit = (plan, shared_constant(which))
-            if len(self._plans) >= 8:
-                self._plans.pop(next(iter(self._plans)))
-            self._plans[key] = hit
-        plan, which = hit
+        from .autograd import Gate, cz_ptm
+        from .windows import layer_blocks
+        plan = _layer_plan(self.n, self.layers, ang.shape[0])
+        which = [(layer // self.block) % self.n_blocks for layer in range(self.layers)]
         cz = cz_ptm(ang.device).reshape(16, 16).contiguous()
         return [Gate(m, q) for m, q in layer_blocks(*gate_ptms(ang, t1, t2), plan, dtype, cz,
                                                     which)]

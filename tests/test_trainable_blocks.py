@@ -1,0 +1,113 @@
+"""TrainableCircuit's blocks built by the library (workloads.TrainableCircuit
+with blocks of three qubits): what the route keeps alive, and the calls it must
+take or leave to the composed gates.  CPU tests run the launches' replays in
+place of the kernels."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from quantumsim_amd import _native as nat
+from quantumsim_amd import windows
+from quantumsim_amd.workloads import TrainableCircuit
+
+# float64 products of at most eight 64 x 64 factors of row sums below 2
+TOL = 8 * 64 * 2 * 2.0 ** -52
+
+
+class _HostLib:
+    """The library with the block kernels' launches replayed on host memory."""
+
+    def __init__(self):
+        self._lib = nat.lib()
+
+    def __getattr__(self, name):
+        return getattr(self._lib, name)
+
+    def qsv_put(self, host, nbytes, dst, stream):
+        ctypes.memmove(dst, host, nbytes)
+        return 0
+
+    def qsv_layer_blocks(self, dtype, n_pos, table, table_dev, batch, n, layers, rot, damp, cz,
+                         out, out_elems, stream):
+        p = lambda a: ctypes.cast(a, nat._c_f64p)
+        return self._lib.qsv_emulate_layer_blocks(n_pos, table_dev, batch, n, layers, p(rot),
+                                                  p(damp), p(cz), p(out), out_elems, None, None,
+                                                  None)
+
+
+@pytest.fixture
+def host_lib(monkeypatch):
+    lib = _HostLib()
+    monkeypatch.setattr(nat, 'lib', lambda: lib)
+    monkeypatch.setattr(windows, '_stream', lambda: None)
+
+
+def _tensors(obj, seen=None):
+    """Tensors reachable from an object's attributes and containers."""
+    seen = set() if seen is None else seen
+    if id(obj) in seen:
+        return []
+    seen.add(id(obj))
+    if isinstance(obj, torch.Tensor):
+        return [obj]
+    if isinstance(obj, dict):
+        return [t for kv in obj.items() for o in kv for t in _tensors(o, seen)]
+    if isinstance(obj, (list, tuple, set)):
+        return [t for o in obj for t in _tensors(o, seen)]
+    return _tensors(vars(obj), seen) if hasattr(obj, '__dict__') else []
+
+
+def _params(tc, sets, device='cpu'):
+    return tc.initial_params(sets, seed=4, device=device, dtype=torch.float64)
+
+
+def test_circuit_object_owns_no_device_memory(host_lib):
+    """Captured launches hold device addresses: none of them may belong to the
+    circuit, which the caller is free to drop or to use with other set counts."""
+    tc = TrainableCircuit(n=5, layers=7)
+    for sets in (1, 2):
+        ang, t1, t2 = _params(tc, sets)
+        got = tc._blocks(ang, t1, t2, torch.float64)
+        ref = tc.gates(ang, t1, t2, 3)
+        assert [g.targets for g in got] == [g.targets for g in ref]
+        for a, b in zip(got, ref):
+            assert (a.ptm - b.ptm).abs().max() <= TOL
+    assert not _tensors(tc)
+
+
+@pytest.mark.gpu
+def test_captured_step_outlives_its_circuit():
+    """Replays of a step whose circuit is gone, after nine other set counts and
+    with the freed memory written over, equal the eager step."""
+    from quantumsim_amd.autograd import capture_step
+
+    def make():
+        tc = TrainableCircuit(n=6, layers=8)
+        params = [p.requires_grad_() for p in _params(tc, 4, 'cuda')]
+        target = torch.full((4, 64), 1 / 64, dtype=torch.float64, device='cuda')
+
+        def step():
+            p = tc.populations(*params, torch.float32, checkpoint_every=4, fuse_qudits=3)
+            return torch.autograd.grad(tc.kl(target, p).sum(), params)
+        # the parameters and the target are the graph's inputs: the caller's to keep
+        return capture_step(step) + ([g.clone() for g in step()], params, target)
+
+    graph, stream, out, ref, *inputs = make()
+    other = TrainableCircuit(n=6, layers=8)
+    for sets in range(5, 14):
+        other.populations(*_params(other, sets, 'cuda'), torch.float32, fuse_qudits=3)
+    del other
+    torch.cuda.synchronize()
+    for rep in range(3):
+        # whatever the allocator has back is handed out and written over
+        junk = [torch.full((size,), 0x7f, dtype=torch.uint8, device='cuda')
+                for size in (512, 2048, 4096, 8192, 1 << 16, 1 << 20) for _ in range(16)]
+        torch.cuda.synchronize()
+        del junk
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, ref):
+            assert torch.equal(a, b), rep
