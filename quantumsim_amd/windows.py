@@ -319,6 +319,9 @@ def layer_blocks(rot, damp, plan, dtype, cz, which=None):
         which = tuple(int(w) for w in (which.tolist() if hasattr(which, 'tolist') else which))
         if len(which) != plan.layers:
             raise ValueError('which must hold one rotation set per layer')
+        for w in which:      # the device's index_select checks nothing
+            if not 0 <= w < sets:
+                raise IndexError('rotation set %d of %d' % (w, sets))
     if plan.device is not None and torch.device(plan.device).type != rot.device.type:
         raise ValueError('a plan for %s, rotation PTMs on %s' % (plan.device, rot.device))
     out = _LayerBlocks.apply(rot, damp, which, plan, dtype, cz)

@@ -111,3 +111,23 @@ def test_captured_step_outlives_its_circuit():
         torch.cuda.synchronize()
         for a, b in zip(out, ref):
             assert torch.equal(a, b), rep
+
+
+@pytest.mark.parametrize('which', [(0, 1, 2), (0, -1, 1)])
+def test_missing_rotation_set_is_refused(host_lib, which):
+    """The layer map indexes the rotation sets on the device, where nothing
+    checks it."""
+    plan = windows.LayerBlockPlan(3, 3, 2)
+    rot = torch.zeros((2, 2, 3, 4, 4), dtype=torch.float64)
+    damp = torch.zeros((2, 3, 4, 4), dtype=torch.float64)
+    cz = torch.zeros((16, 16), dtype=torch.float64)
+    with pytest.raises(IndexError, match='rotation set'):
+        windows.layer_blocks(rot, damp, plan, torch.float64, cz, which)
+
+
+def test_fewer_rotation_sets_than_blocks(host_lib):
+    tc = TrainableCircuit(n=4, layers=12, block=4, n_blocks=3)
+    ang, t1, t2 = _params(tc, 2)
+    for make in (lambda a: tc.gates(a, t1, t2, 3), lambda a: tc._blocks(a, t1, t2, torch.float64)):
+        with pytest.raises(IndexError):
+            make(ang[:, :2].contiguous())
