@@ -118,7 +118,9 @@ class LayerBlockPlan:
     (offset of the first part, of the second)).  Host memory only:
     layer_blocks writes the table to the device in every call, so that a
     captured step depends on no plan's lifetime.  ``device``: the only one the
-    plan is used on (None: any)."""
+    plan is used on (None: any).  NotImplementedError where a block holds more
+    than eight gates (up to three qubits and a few layers on: all of them are one
+    block), the split blocks differ in size, or there is nothing to build."""
 
     def __init__(self, n, layers, batch, device=None):
         self.n, self.layers, self.batch = n, layers, batch
@@ -126,13 +128,15 @@ class LayerBlockPlan:
         layer_of = [layer for layer in range(layers) for _ in layer_targets(n, layer)]
         plan = fuse_plan(gates, [4] * n, 3)
         if any(len(src) > 8 for _, src in plan):
-            raise ValueError('a block of more than eight gates')
+            raise NotImplementedError('a block of more than eight gates')
         whole = [k for k, (_, src) in enumerate(plan) if len(src) <= 4]
         split = [k for k, (_, src) in enumerate(plan) if len(src) > 4]
         if len({len(plan[k][0]) for k in split}) > 1:
-            raise ValueError('split blocks of several sizes')
+            raise NotImplementedError('split blocks of several sizes')
         parts = [(k, plan[k][1]) for k in whole] + [(k, plan[k][1][:4]) for k in split] + \
                 [(k, plan[k][1][4:]) for k in split]
+        if not (1 <= len(parts) <= 65535 and 1 <= batch <= 65535):    # the launch's grid
+            raise NotImplementedError('%d blocks for %d sets' % (len(parts), batch))
         self.table = np.zeros(len(parts), WBLOCK_DTYPE)
         self.blocks = [(tuple(qs), 4 ** len(qs)) for qs, _ in plan]
         self.offset = {}                 # whole block -> offset

@@ -333,9 +333,13 @@ def _gate_ptms_function():
 
 @functools.lru_cache(maxsize=32)
 def _layer_plan(n, layers, sets):
-    """windows.LayerBlockPlan, kept for the circuits last used (host memory)."""
+    """windows.LayerBlockPlan, or None where it takes no such circuit; kept for
+    the circuits last used (host memory)."""
     from .windows import LayerBlockPlan
-    return LayerBlockPlan(n, layers, sets)
+    try:
+        return LayerBlockPlan(n, layers, sets)
+    except NotImplementedError:
+        return None
 
 
 class TrainableCircuit:
@@ -377,10 +381,18 @@ class TrainableCircuit:
             out = [Gate(m, q) for m, q in fuse_batched(out, [4] * self.n, fuse_qudits)]
         return out
 
+    @staticmethod
+    def _on_device(*tensors):
+        return all(t.is_cuda for t in tensors)
+
     def _blocks(self, ang, t1, t2, dtype):
+        """The blocks gates() composes, built by the library in one launch; None
+        for the circuits it does not take (windows.LayerBlockPlan)."""
         from .autograd import Gate, cz_ptm
         from .windows import layer_blocks
         plan = _layer_plan(self.n, self.layers, ang.shape[0])
+        if plan is None:
+            return None
         which = [(layer // self.block) % self.n_blocks for layer in range(self.layers)]
         cz = cz_ptm(ang.device).reshape(16, 16).contiguous()
         return [Gate(m, q) for m, q in layer_blocks(*gate_ptms(ang, t1, t2), plan, dtype, cz,
@@ -394,10 +406,11 @@ class TrainableCircuit:
         N = 4 ** self.n
         x0 = torch.zeros((S, N), dtype=dtype, device=ang.device)
         x0[:, 0] = 1
-        if fuse_qudits == 3 and ang.dtype == t1.dtype == t2.dtype == torch.float64:
-            # the blocks gates() composes, built by the library in one launch
+        gates = None
+        if fuse_qudits == 3 and ang.dtype == t1.dtype == t2.dtype == torch.float64 and \
+                self._on_device(ang, t1, t2):
             gates = self._blocks(ang, t1, t2, dtype)
-        else:
+        if gates is None:
             gates = self.gates(ang, t1, t2, fuse_qudits)
         x = run_circuit(x0, gates, (4,) * self.n, checkpoint_every)
         return diagonal(x, [general(2)] * self.n)

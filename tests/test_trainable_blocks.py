@@ -131,3 +131,58 @@ def test_fewer_rotation_sets_than_blocks(host_lib):
     for make in (lambda a: tc.gates(a, t1, t2, 3), lambda a: tc._blocks(a, t1, t2, torch.float64)):
         with pytest.raises(IndexError):
             make(ang[:, :2].contiguous())
+
+
+@pytest.fixture
+def gates_of(host_lib, monkeypatch):
+    """The gates that populations() hands to run_circuit, on host tensors."""
+    from quantumsim_amd import autograd
+    seen = []
+
+    def run_circuit(x0, gates, shape, checkpoint_every):
+        seen.append(gates)
+        return x0
+    monkeypatch.setattr(autograd, 'run_circuit', run_circuit)
+    monkeypatch.setattr(autograd, 'diagonal', lambda x, bases: x)
+    # the library's route is for tensors on a device; the replay takes host ones
+    monkeypatch.setattr(TrainableCircuit, '_on_device', staticmethod(lambda *t: True),
+                        raising=False)
+
+    def call(tc, ang, t1, t2):
+        tc.populations(ang, t1, t2, torch.float64, fuse_qudits=3)
+        return seen.pop()
+    return call
+
+
+def _same_gates(got, ref):
+    assert [g.targets for g in got] == [g.targets for g in ref]
+    for a, b in zip(got, ref):
+        assert a.ptm.shape == b.ptm.shape
+        # float64 products of up to 80 factors of row sums below 2, damped
+        assert ((a.ptm - b.ptm).abs() <= 10 * TOL).all()
+
+
+@pytest.mark.parametrize('n,layers', [(1, 9), (1, 40), (2, 6), (2, 40), (3, 5), (3, 40), (4, 40),
+                                      (5, 0), (4, 1), (6, 12)])
+def test_every_width_and_depth(gates_of, n, layers):
+    """Few qubits put all the layers' gates into one block."""
+    tc = TrainableCircuit(n=n, layers=layers)
+    for sets in (0, 1, 3):
+        p = _params(tc, sets)
+        _same_gates(gates_of(tc, *p), tc.gates(*p, 3))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,layers', [(1, 40), (2, 6), (3, 5), (3, 40), (4, 40)])
+def test_populations_of_few_qubits(n, layers):
+    """Populations and gradients in blocks against one gate at a time, float64."""
+    tc = TrainableCircuit(n=n, layers=layers)
+    out = []
+    for fuse in (3, 0):
+        p = [t.requires_grad_() for t in _params(tc, 2, 'cuda')]
+        pops = tc.populations(*p, torch.float64, fuse_qudits=fuse)
+        w = torch.linspace(-1, 1, pops.numel(), dtype=torch.float64, device='cuda').view_as(pops)
+        out.append([pops.detach()] + list(torch.autograd.grad((pops * w).sum(), p)))
+    for a, b in zip(*out):
+        # up to 2 x 40 applications, 64 products of entries below 2 each
+        assert (a - b).abs().max().item() <= 80 * 64 * 2 * 2.0 ** -52 * max(1.0, b.abs().max().item())
