@@ -186,3 +186,16 @@ def test_populations_of_few_qubits(n, layers):
     for a, b in zip(*out):
         # up to 2 x 40 applications, 64 products of entries below 2 each
         assert (a - b).abs().max().item() <= 80 * 64 * 2 * 2.0 ** -52 * max(1.0, b.abs().max().item())
+
+
+def test_shared_and_wider_parameters(gates_of):
+    """What the composition broadcasts or ignores: T1 and T2 or angles shared by
+    the sets, parameters of more qubits, sets or layers of angles than are used."""
+    tc = TrainableCircuit(n=4, layers=7)
+    ang, t1, t2 = _params(tc, 3)
+    wide = TrainableCircuit(n=5, layers=7, n_blocks=4)
+    wang, w1, w2 = _params(wide, 3)
+    for p in [(ang, t1[:1], t2[:1]), (ang[:1], t1, t2), (ang[:1], t1[:1], t2[:1]),
+              (wang, w1, w2), (ang, w1, w2), (wang, t1, t2),
+              (ang.transpose(0, 1).contiguous().transpose(0, 1), t1, t2)]:
+        _same_gates(gates_of(tc, *p), tc.gates(*p, 3))
