@@ -388,10 +388,12 @@ class TrainableCircuit:
     def _blocks(self, ang, t1, t2, dtype):
         """The blocks gates() composes, built by the library in one launch; None
         for parameters shared by the sets or of more qubits than the circuit's
-        (the composition broadcasts and ignores them) and for the circuits it
-        does not take (windows.LayerBlockPlan)."""
+        (the composition broadcasts and ignores them), for gates() overridden
+        and for the circuits it does not take (windows.LayerBlockPlan)."""
         from .autograd import Gate, cz_ptm
         from .windows import layer_blocks
+        if getattr(self.gates, '__func__', None) is not TrainableCircuit.gates:
+            return None
         if ang.dim() != 4 or ang.shape[2:] != (self.n, 2) or \
                 not t1.shape == t2.shape == (ang.shape[0], self.n):
             return None

@@ -199,3 +199,23 @@ def test_shared_and_wider_parameters(gates_of):
               (wang, w1, w2), (ang, w1, w2), (wang, t1, t2),
               (ang.transpose(0, 1).contiguous().transpose(0, 1), t1, t2)]:
         _same_gates(gates_of(tc, *p), tc.gates(*p, 3))
+
+
+def test_overridden_gates_are_used(gates_of):
+    """gates() is the circuit's definition: a subclass's or an instance's own is
+    what populations() runs."""
+    class Reversed(TrainableCircuit):
+        def gates(self, ang, t1, t2, fuse_qudits=0):
+            return super().gates(ang, t1, t2, fuse_qudits)[::-1]
+
+    tc = Reversed(n=4, layers=7)
+    p = _params(tc, 2)
+    _same_gates(gates_of(tc, *p), tc.gates(*p, 3))
+    tc = TrainableCircuit(n=4, layers=7)
+    plain = tc.gates(*p, 3)
+    tc.gates = lambda ang, t1, t2, fuse_qudits=0: plain[:2]
+    _same_gates(gates_of(tc, *p), plain[:2])
+
+    class Renamed(TrainableCircuit):         # the same gates: either route
+        pass
+    _same_gates(gates_of(Renamed(n=4, layers=7), *p), plain)
