@@ -384,7 +384,9 @@ int64_t qsv_ptm_grad_noalloc_scratch_bytes(void);
  * ybar x^T as qsv_ptm_grad computes it; reads x and ybar once and writes
  * xbar (three streams instead of four).  xbar is bitwise the transposed
  * apply's (the same k-steps of four entries in the same order).  workspace:
- * qsv_ptm_grad_workspace_bytes of the same geometry.  QSV_ENOTSUP unless the
+ * at least qsv_ptm_grad_workspace_bytes of the same geometry; with
+ * qsv_batched_backward_workspace_bytes a few large float32 states are split
+ * over more blocks (dptm differs in the order of its float64 sums).  QSV_ENOTSUP unless the
  * states are 16-byte aligned and, for float64, the innermost axis is a
  * unit-stride bystander; for float32, the tiles of 32 orbits are whole and
  * either the orbits come in 4-orbit vectors (innermost axis a bystander)
@@ -398,6 +400,10 @@ int qsv_apply_ptm_batched_backward(int dtype, const void* x, const void* ybar, v
                                    const int32_t* targets, const void* ptm_dev,
                                    int64_t ptm_batch_stride, void* dptm, int accumulate,
                                    void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Bytes of device workspace qsv_apply_ptm_batched_backward makes use of. */
+int64_t qsv_batched_backward_workspace_bytes(int dtype, int batch, int rank, const int64_t* dims,
+                                             int k, const int32_t* targets);
 
 /* QSV_OK if qsv_apply_ptm_batched_backward takes this geometry (its states
  * aligned), QSV_ENOTSUP if not. */
@@ -417,7 +423,8 @@ int qsv_batched_backward_applies(int dtype, int rank, const int64_t* dims, int k
  *     aligned states take qsv_apply_ptm_batched_backward, others
  *     qsv_ptm_grad_tiled and the apply with ptm_t, the transposed PTMs.
  *     workspace: at least every position's `workspace` bytes (what
- *     qsv_ptm_grad_workspace_bytes gives for `active`); with more, the final
+ *     qsv_ptm_grad_workspace_bytes gives for `active`, for `fused` ones
+ *     qsv_batched_backward_workspace_bytes); with more, the final
  *     sums of up to sixteen gradients share a launch (without a hook).
  * hook (may be NULL): called before (phase 0) and after (phase 1) each launch
  * with its kind, position and batch.  Same launches as the single calls;

@@ -88,6 +88,8 @@ _SIGNATURES = {
     'qsv_emulate_ptm_grad': (ctypes.c_int, [ctypes.c_int, _c_f64p, _c_f64p, ctypes.c_int, _c_i64p,
                                             ctypes.c_int, _c_i32p, _c_i32p, _c_f64p,
                                             ctypes.c_int32, _c_i32p]),
+    'qsv_batched_backward_workspace_bytes': (ctypes.c_int64, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, _c_i64p, ctypes.c_int, _c_i32p]),
     'qsv_batched_backward_applies': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _c_i64p,
                                                     ctypes.c_int, _c_i32p]),
     'qsv_schedule_forward': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _c_i64p, ctypes.c_int,

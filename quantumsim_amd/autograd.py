@@ -141,10 +141,10 @@ def _fused_backward_raw(x, gy, ptm, shape, targets, gx_out=None, gp_out=None):
     if any(t.data_ptr() % 16 for t in (x, gy, gx)):
         return None
     L = nat.lib()
-    d = [shape[q] for q in targets]
     pstride = 0 if ptm.shape[0] == 1 else 64 * 64
-    ws = nat.check(L.qsv_ptm_grad_workspace_bytes(B, len(shape), nat.i64(shape), len(targets),
-                                                  nat.i32(targets), nat.i32(d)), 'backward')
+    ws = nat.check(L.qsv_batched_backward_workspace_bytes(
+        nat.dtype_code(x.dtype), B, len(shape), nat.i64(shape), len(targets),
+        nat.i32(targets)), 'backward')
     buf = _Workspace.get(x.device, ws)
     gp = torch.empty((B, 64, 64), dtype=x.dtype, device=x.device) if gp_out is None else gp_out
     assert gp.shape[0] >= B and tuple(gp.shape[1:]) == (64, 64) and gp.is_contiguous()
@@ -359,9 +359,12 @@ class _SchedulePositions:
                 r.has_grad = tile is not None
                 if tile is not None:
                     r.grad = tile
-                r.workspace = nat.check(L.qsv_ptm_grad_workspace_bytes(
-                    active, len(self.shape), nat.i64(self.shape), len(tg), nat.i32(tg),
-                    nat.i32(d)), 'ptm_grad')
+                dims, k, t = nat.i64(self.shape), len(tg), nat.i32(tg)
+                r.workspace = nat.check(
+                    L.qsv_batched_backward_workspace_bytes(
+                        nat.dtype_code(dtype), active, len(self.shape), dims, k, t) if r.fused else
+                    L.qsv_ptm_grad_workspace_bytes(active, len(self.shape), dims, k, t,
+                                                   nat.i32(d)), 'ptm_grad')
                 most = max(most, r.workspace)
         return most
 

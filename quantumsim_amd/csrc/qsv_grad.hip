@@ -1724,9 +1724,21 @@ extern "C" int64_t qsv_ptm_grad_workspace_bytes(int batch, int rank, const int64
   GradPlan p;
   const int rc = make_grad_plan(8, rank, dims, k, targets, dims_out_t, p);
   if (rc) return rc;
-  int64_t blocks = int64_t(batch) * max_grad_blocks(p);
-  if (p.din == 64 && p.dout == 64 && batch > 0) blocks = std::max<int64_t>(blocks, kBwdBlocks);
-  return blocks * p.din * p.dout * 8;
+  return int64_t(batch) * max_grad_blocks(p) * p.din * p.dout * 8;
+}
+
+extern "C" int64_t qsv_batched_backward_workspace_bytes(int dtype, int batch, int rank,
+                                                        const int64_t* dims, int k,
+                                                        const int32_t* targets) {
+  QSV_CHECK_ARG(dtype == QSV_F32 || dtype == QSV_F64, "unknown dtype %d", dtype);
+  QSV_CHECK_ARG(dims && targets && k >= 1 && k <= QSV_MAX_TARGETS, "bad target list");
+  int32_t dout[QSV_MAX_TARGETS];
+  for (int j = 0; j < k; ++j) {
+    QSV_CHECK_ARG(targets[j] >= 0 && targets[j] < rank, "target %d does not exist", targets[j]);
+    dout[j] = int32_t(dims[targets[j]]);
+  }
+  const int64_t least = qsv_ptm_grad_workspace_bytes(batch, rank, dims, k, targets, dout);
+  return dtype == QSV_F32 && least > 0 ? std::max<int64_t>(least, kBwdBlocks * 64 * 64 * 8) : least;
 }
 
 template <typename T>
@@ -2520,22 +2532,23 @@ static int bwd64_blocks(const GradPlan& p, int batch, uint32_t cap) {
 // k_bwd64d / k_bwd64q: block groups, one round of resident blocks over the batch
 // (occupancy x CUs / batch per state), at least 4 tiles per group and at most
 // kGrad64Blocks.  A group is split (whole float32 partial sums each) until the
-// launch has kBwdBlocks blocks: two 11-qubit circuits make 128 groups for 256
+// launch has `most` blocks, kBwdBlocks or as many as the workspace holds the
+// partials of: two 11-qubit circuits make 128 groups for 256
 // compute units, and their training step took 12.5 ms, 8.0 ms with four blocks a
 // group; from six circuits (two blocks a group) on it makes no difference.
-static BwdTiles bwd64_split(uint32_t tiles, uint32_t stride, uint32_t batch) {
+static BwdTiles bwd64_split(uint32_t tiles, uint32_t stride, uint32_t batch, uint32_t most) {
   BwdTiles r;
   r.stride = stride;
   const uint32_t sums = ((tiles + stride - 1) / stride + kDirFlush - 1) / kDirFlush;
   const uint32_t parts = std::max<uint32_t>(
-      1, std::min<uint32_t>(sums, kBwdBlocks / std::max<uint32_t>(1, stride * batch)));
+      1, std::min<uint32_t>(sums, most / std::max<uint32_t>(1, stride * batch)));
   const uint32_t each = std::max<uint32_t>(1, (sums + parts - 1) / parts);
   r.parts = std::max<uint32_t>(1, (sums + each - 1) / each);
   r.run = each * kDirFlush;
   return r;
 }
 
-static BwdTiles bwd64_tiles(const GradPlan& p, int batch) {
+static BwdTiles bwd64_tiles(const GradPlan& p, int batch, int64_t workspace_bytes) {
   static const uint32_t cap_d =
       resident_blocks(reinterpret_cast<const void*>(k_bwd64d<true>));
   static const uint32_t cap_q =
@@ -2544,7 +2557,8 @@ static BwdTiles bwd64_tiles(const GradPlan& p, int batch) {
   const uint32_t tiles = p.n_orbits / kDirTile;
   return bwd64_split(
       tiles,
-      std::max<uint32_t>(1, std::min<uint32_t>(std::min(cap / B, tiles / 4), kGrad64Blocks)), B);
+      std::max<uint32_t>(1, std::min<uint32_t>(std::min(cap / B, tiles / 4), kGrad64Blocks)), B,
+      uint32_t(std::max<int64_t>(0, std::min<int64_t>(kBwdBlocks, workspace_bytes / (64 * 64 * 8)))));
 }
 
 template <typename T, int VN>
@@ -2594,7 +2608,7 @@ static int batched_backward_run(int dtype, const void* x, const void* ybar, void
   const FusedOffs fo = bwd64_offsets(p);
   // bwd64_plan admits only k_bwd64d's and k_bwd64q's float32 geometries
   const bool direct = dtype == QSV_F32;
-  const BwdTiles tiles = direct ? bwd64_tiles(p, batch) : BwdTiles{1, 1, 1};
+  const BwdTiles tiles = direct ? bwd64_tiles(p, batch, workspace_bytes) : BwdTiles{1, 1, 1};
   const int nb = direct ? int(tiles.stride * tiles.parts)
                         : bwd64_blocks(p, batch, bwd64_cap<double, 2>());
   const int64_t need = int64_t(batch) * nb * 64 * 64 * 8;
@@ -2943,7 +2957,7 @@ extern "C" int qsv_emulate_apply_ptm_batched_backward(int dtype, const double* x
   if (dtype == QSV_F32) {  // bwd64_plan admits only k_bwd64d's and k_bwd64q's geometries
     const BwdTiles tiles = bwd64_split(
         p.n_orbits / kDirTile,
-        uint32_t(grad_blocks > 0 ? grad_blocks : grad64_blocks(p.n_orbits, 1)), 1);
+        uint32_t(grad_blocks > 0 ? grad_blocks : grad64_blocks(p.n_orbits, 1)), 1, kBwdBlocks);
     return p.quad ? emulate_bwd64q(p, x, ybar, tiles, dptm, ptm, xbar)
                   : emulate_grad64d(p, x, ybar, tiles, dptm, ptm, xbar);
   }
