@@ -281,7 +281,8 @@ class QubitBlocks:
 
 def _qubit_gates(gates, n):
     """(ks, targets, ptms) arrays of a circuit of 1- and 2-qubit gates with
-    real square PTMs on n qubits, or None if it holds any other gate."""
+    real, finite square PTMs on n qubits, or None if it holds any other gate
+    (the library skips zeros where ``fuse`` makes 0 * inf a NaN)."""
     ks, targets, ptms = [], [], []
     for ptm, qudits in gates:
         p = np.asarray(ptm)
@@ -294,8 +295,10 @@ def _qubit_gates(gates, n):
         ks.append(k)
         targets += q if k == 2 else (q[0], -1)
         ptms.append(p.reshape(-1))
-    return (np.array(ks, dtype=np.int32), np.array(targets, dtype=np.int32),
-            np.concatenate(ptms).astype(np.float64, copy=False))
+    flat = np.concatenate(ptms).astype(np.float64, copy=False)
+    if not np.isfinite(flat).all():
+        return None
+    return np.array(ks, dtype=np.int32), np.array(targets, dtype=np.int32), flat
 
 
 def _native_circuit(pv, gates):
