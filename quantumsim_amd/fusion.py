@@ -329,7 +329,7 @@ def apply_circuit(pv, gates, max_qudits=3):
         for ptm, qudits in gates:
             pv.apply_ptm(np.asarray(ptm), *qudits)
         return len(gates)
-    gates = list(gates)
+    gates = [(ptm, tuple(qudits)) for ptm, qudits in gates]
     arrays = _native_circuit(pv, gates) if gates else None
     if arrays is None:
         fused = fuse(gates, list(pv.dim_pauli), max_qudits)

@@ -53,3 +53,16 @@ def test_non_finite_ptms(applied, value, order):
     for (p, _), f in zip(got, ref):
         np.testing.assert_array_equal(np.isnan(p), np.isnan(f.ptm))
         np.testing.assert_array_equal(np.isinf(p), np.isinf(f.ptm))
+
+
+def test_targets_of_any_iterable(applied):
+    """Targets are read once, as fuse() reads them."""
+    rng = np.random.default_rng(3)
+    qs = [(0, 1), (2, 3), (1, 2)]
+    ptms = [rng.standard_normal((4,) * 4) for _ in qs]
+    ref = fuse(list(zip(ptms, qs)), [4] * 4, 3)
+    for third in (rng.standard_normal((4,) * 4), rng.standard_normal((4,) * 6)):
+        tail = tuple(range(third.ndim // 2))
+        got = applied(4, iter([(p, iter(q)) for p, q in zip(ptms + [third], qs + [tail])]))
+        ref = fuse(list(zip(ptms + [third], qs + [tail])), [4] * 4, 3)
+        assert [q for _, q in got] == [f.qudits for f in ref]
