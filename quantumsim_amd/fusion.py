@@ -334,7 +334,7 @@ def apply_circuit(pv, gates, max_qudits=3):
     if arrays is None:
         fused = fuse(gates, list(pv.dim_pauli), max_qudits)
     else:
-        fused = QubitBlocks(pv.n_qubits, *arrays, max_qudits)
+        fused = QubitBlocks(pv.n_qubits, *arrays, min(max_qudits, pv.n_qubits))
         if len(fused) > 1 and pv.run_passes(*arrays):
             return len(fused)
     for ptm, qudits in fused:

@@ -55,6 +55,17 @@ def test_non_finite_ptms(applied, value, order):
         np.testing.assert_array_equal(np.isinf(p), np.isinf(f.ptm))
 
 
+@pytest.mark.parametrize('max_qudits', [float('inf'), 2.5, 4.0])
+def test_bound_of_any_number(applied, max_qudits):
+    rng = np.random.default_rng(2)
+    gates = [(rng.standard_normal((4,) * 4), (q, q + 1)) for q in (0, 2, 1)]
+    ref = fuse(gates, [4] * 4, max_qudits)
+    got = applied(4, gates, max_qudits)
+    assert [q for _, q in got] == [f.qudits for f in ref]
+    for (p, _), f in zip(got, ref):
+        np.testing.assert_allclose(p, f.ptm, rtol=0, atol=1e-12)
+
+
 def test_targets_of_any_iterable(applied):
     """Targets are read once, as fuse() reads them."""
     rng = np.random.default_rng(3)
