@@ -213,7 +213,8 @@ int qsv_circuits_forward(int dtype, int n_circuits, const qsv_circuit* circs_dev
  *   qsv_circuit_create   composes the gates into two-qubit blocks and plans
  *                        the passes (host memory only); *plan_out is freed
  *                        with qsv_circuit_destroy.  QSV_ENOTSUP: strides the
- *                        passes cannot read in aligned runs.
+ *                        passes cannot read in aligned runs (the innermost
+ *                        axis not of stride 1 among them).
  *   qsv_circuit_passes   number of passes
  *   qsv_circuit_table    writes the blocks' tables (qsv_circuit_table_bytes)
  *                        to host memory; the caller copies them to the device

@@ -884,8 +884,9 @@ extern "C" int qsv_circuit_create(int n_qubits, const int64_t* strides, int n_ga
   for (int q = n_qubits - 1; q >= 0; --q) {
     QSV_CHECK_ARG(strides[q] >= acc && strides[q] < (int64_t(1) << 40),
                   "strides of axis %d overlap the axes below it", q);
-    // runs of whole 16-byte vectors: the lowest bits nest without a gap
-    if (strides[q] < 8 ? strides[q] != acc : strides[q] % 8 != 0) {
+    // runs of whole 16-byte vectors: the innermost axis has stride 1 and the lowest
+    // bits nest without a gap
+    if (strides[q] < 8 || q == n_qubits - 1 ? strides[q] != acc : strides[q] % 8 != 0) {
       set_error("circuit passes need axes that nest in aligned runs of 64 bytes");
       return QSV_ENOTSUP;
     }

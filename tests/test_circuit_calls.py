@@ -3,8 +3,9 @@ leave alone or treat as the composition on the host does (quantumsim_amd.fusion)
 import numpy as np
 import pytest
 
+from quantumsim_amd import _native as nat
 from quantumsim_amd import fusion
-from quantumsim_amd.fusion import _qubit_gates, fuse
+from quantumsim_amd.fusion import CircuitPasses, _qubit_gates, fuse
 
 
 class _Recorder:
@@ -77,3 +78,36 @@ def test_targets_of_any_iterable(applied):
         got = applied(4, iter([(p, iter(q)) for p, q in zip(ptms + [third], qs + [tail])]))
         ref = fuse(list(zip(ptms + [third], qs + [tail])), [4] * 4, 3)
         assert [q for _, q in got] == [f.qudits for f in ref]
+
+
+@pytest.mark.parametrize('strides', [[128, 32, 8], [512, 128, 16], [32, 8, 2], [16, 8, 1]])
+def test_strides_without_a_unit_axis_are_refused(strides):
+    """The passes read pairs of neighbouring entries: the innermost axis has
+    stride 1 (and no axis overlaps another)."""
+    rng = np.random.default_rng(0)
+    arrays = _qubit_gates([(rng.standard_normal((4,) * 4), (0, 1))], 3)
+    with pytest.raises((NotImplementedError, ValueError)):
+        CircuitPasses(3, strides, *arrays)
+
+
+@pytest.mark.parametrize('n,pad_from', [(4, 2), (5, 2), (7, 3), (9, 5), (10, 4)])
+def test_replay_of_padded_layouts(n, pad_from):
+    """Axes from some on padded by 4 KB, as large vectors have them."""
+    from test_circuit_passes import _apply, _circuit, _strides
+    rng = np.random.default_rng(30 * n)
+    for kind in ('brick', 'random'):
+        gates = _circuit(n, kind, rng)
+        x = rng.standard_normal((4,) * n)
+        strides, extent = _strides(n, pad_from, 512)
+        assert extent > x.size
+        phys = np.full(extent, np.nan)
+        view = np.lib.stride_tricks.as_strided(phys, x.shape, [8 * s for s in strides])
+        view[...] = x
+        plan = CircuitPasses(n, strides, *_qubit_gates(gates, n))
+        nat.check(nat.lib().qsv_emulate_circuit(plan.handle, phys.ctypes.data_as(nat._c_f64p)),
+                  'run')
+        # 16 products and sums per gate, each within half an ulp of a norm that
+        # the gates keep
+        ref = _apply(x, gates)
+        assert np.linalg.norm(view - ref) <= 32 * len(gates) * 2.0 ** -53 * np.linalg.norm(x)
+        assert np.isnan(phys).sum() == extent - x.size
