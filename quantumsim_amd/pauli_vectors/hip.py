@@ -180,6 +180,8 @@ class PauliVectorHIP(PauliVectorBase):
     """
 
     _diag_plans = OrderedDict()
+    # what a vector keeps for its own next call, and no copy takes over
+    _geo = (None, None, None, None)      # _geometry()'s arrays and their layout
 
     def __init__(self, bases, pv=None, *, force=False, dtype=None, device=None):
         super().__init__(bases, pv, force=force)
@@ -218,10 +220,16 @@ class PauliVectorHIP(PauliVectorBase):
         store._qsv_home = _raw_stream(self._device)
         self._store = store           # owning storage of the state
         self._data = store            # physical (padded) extent
-        self._geo = (None, None, None, None)
         self._spare = None            # second buffer (apply_ptm writes there)
 
     # ------------------------------------------------------------ plumbing
+    def __getstate__(self):
+        """For the copy and pickle modules: without the library's argument
+        arrays, which they cannot save."""
+        state = dict(self.__dict__)
+        state.pop('_geo', None)
+        return state
+
     @property
     def dtype(self):
         return self._dtype
