@@ -182,6 +182,7 @@ class PauliVectorHIP(PauliVectorBase):
     _diag_plans = OrderedDict()
     # what a vector keeps for its own next call, and no copy takes over
     _geo = (None, None, None, None)      # _geometry()'s arrays and their layout
+    _store_home = _spare_home = None     # streams that allocated the buffers
 
     def __init__(self, bases, pv=None, *, force=False, dtype=None, device=None):
         super().__init__(bases, pv, force=force)
@@ -217,17 +218,19 @@ class PauliVectorHIP(PauliVectorBase):
             view.copy_(pv.detach().to(device=self._device, dtype=self._dtype))
         else:
             view[(0,) * len(self._shape)] = 1
-        store._qsv_home = _raw_stream(self._device)
         self._store = store           # owning storage of the state
+        self._store_home = _raw_stream(self._device)
         self._data = store            # physical (padded) extent
         self._spare = None            # second buffer (apply_ptm writes there)
 
     # ------------------------------------------------------------ plumbing
     def __getstate__(self):
         """For the copy and pickle modules: without the library's argument
-        arrays, which they cannot save."""
+        arrays, which they cannot save, and the buffers' streams, which are
+        not the copies'."""
         state = dict(self.__dict__)
-        state.pop('_geo', None)
+        for name in ('_geo', '_store_home', '_spare_home'):
+            state.pop(name, None)
         return state
 
     @property
@@ -261,24 +264,28 @@ class PauliVectorHIP(PauliVectorBase):
         go back to that stream's pool when it is dropped (a spare replaced by
         a larger one, the vector deleted) and could be handed out again while
         this stream's kernels still read or write it; the caching allocator
-        ignores the mark for a buffer's own allocation stream, so buffers
-        known to be this stream's (_qsv_home) are not marked."""
+        ignores the mark for a buffer's own allocation stream, so the vector's
+        own of this stream (_store_home, _spare_home) are not marked."""
         raw = _raw_stream(self._device)
         for t in tensors:
-            if t is not None and getattr(t, '_qsv_home', None) != raw:
+            home = self._store_home if t is self._store else \
+                self._spare_home if t is self._spare else None
+            if t is not None and home != raw:
                 t.record_stream(torch.cuda.current_stream(self._device))
 
     def _take_spare(self, n):
         sp = self._spare
         if sp is None or sp.numel() < n:
             sp = torch.empty(max(n, 1), dtype=self._dtype, device=self._device)
-            sp._qsv_home = _raw_stream(self._device)
+            self._spare_home = _raw_stream(self._device)
         self._spare = None
         return sp
 
     def _swap_in(self, store, extent, shape, strides):
+        """``store``, taken from _take_spare, becomes the state."""
         self._spare = self._store
         self._store = store
+        self._store_home, self._spare_home = self._spare_home, self._store_home
         self._data = store if store.numel() == extent else store[:extent]
         self._shape = tuple(shape)
         self._pstr = tuple(strides)
@@ -368,8 +375,8 @@ class PauliVectorHIP(PauliVectorBase):
         if rc != 0:
             self._spare = out
             nat.check(rc, 'apply_ptm')
-        self._used_here(self._store, out)
         self._swap_in(out, extent, new_shape, new_str)
+        self._used_here(self._store, self._spare)
 
     def run_passes(self, ks, targets, ptms):
         """Apply a circuit of 1- and 2-qubit gates (fusion.CircuitPasses'
@@ -395,8 +402,8 @@ class PauliVectorHIP(PauliVectorBase):
         except Exception:
             self._spare = out
             raise
-        self._used_here(self._store, out)
         self._swap_in(out, extent, self._shape, self._pstr)
+        self._used_here(self._store, self._spare)
         return True
 
     # ------------------------------------------------------------ readouts

@@ -50,6 +50,20 @@ def test_vectors_are_copied_and_saved(monkeypatch):
         assert list(dims) == [4, 4, 4] and list(strides) == list(pv._pstr)
 
 
+def test_copies_do_not_take_over_the_home_stream(monkeypatch):
+    """A copy's buffers belong to the stream that made the copy: until they are
+    known to be of the current stream, their use there is marked."""
+    pv = _vector(monkeypatch, stream=7)
+    new = copy.deepcopy(pv)                     # as if made under another stream
+    monkeypatch.setattr(torch.cuda, 'current_stream', lambda device=None: None)
+    marked = []
+    monkeypatch.setattr(torch.Tensor, 'record_stream', lambda t, s: marked.append(t))
+    pv._used_here(pv._store, pv._spare)
+    assert not marked                           # made on the stream that uses them
+    new._used_here(new._store, new._spare)
+    assert len(marked) == 2
+
+
 @pytest.mark.gpu
 def test_device_vectors_are_copied_and_saved():
     rng = np.random.default_rng(0)
