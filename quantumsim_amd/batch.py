@@ -171,6 +171,9 @@ class CircuitBatch:
         circuits = []
         for gi in self.small:
             g = self.groups[gi]
+            if g.layers[0] == 0:             # no gates, and no part of the pool
+                circuits += [(g.n, [])] * len(g.members)
+                continue
             plan = self._pool_plan(gi)
             B, n0 = len(g.members), len(layer_targets(g.n, 0))
             by_parity = [plan.positions[:n0], plan.positions[n0:]]
@@ -196,6 +199,8 @@ class CircuitBatch:
         cz = self._cached(('cz16',), lambda: cz_ptm(self.device).reshape(16, 16).contiguous())
         for gi in self.small:
             g = self.groups[gi]
+            if g.layers[0] == 0:
+                continue
             plan = self._pool_plan(gi)
             keep8 = self._cached(('keepall', gi), lambda: torch.ones(
                 (plan.batch, plan.nw), dtype=torch.uint8, device=self.device))

@@ -275,7 +275,8 @@ def gate_ptms(angles, t1, t2, layers=None):
     layers = angles.shape[1] if layers is None else layers
     if not (angles.is_cuda and angles.dtype == t1.dtype == t2.dtype == torch.float64
             and angles.device == t1.device == t2.device and angles.dim() == 4
-            and angles.shape[3] == 2 and t1.shape == t2.shape == angles[:, 0, :, 0].shape):
+            and angles.shape[3] == 2
+            and t1.shape == t2.shape == (angles.shape[0], angles.shape[2])):
         return _gate_ptms_ops(angles, t1, t2, layers)
     return _gate_ptms_function().apply(angles, t1, t2, layers)
 
