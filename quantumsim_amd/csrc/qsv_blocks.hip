@@ -37,6 +37,7 @@ constexpr int kWB = 256;  // threads per workgroup
 struct WBGeom {
   int batch, nw, n, layers;  // circuits, windows, qubits, rotation layers
   int span;                  // layers per window
+  int first;                 // window of the launch's blockIdx.y = 0
   const double* rot;         // [batch][layers][n][4][4]
   const double* damp;        // [batch][n][4][4]
   const uint8_t* keep;       // [batch][nw], or NULL: every layer is kept
@@ -391,7 +392,7 @@ __global__ void __launch_bounds__(kWB)
                     int64_t out_elems) {
   constexpr int NF = ONE ? 1 : 4, MD = ONE ? 16 : 64;
   __shared__ double F[NF * 256], Tm[NF * 256], M[MD * MD];
-  const int b = blockIdx.x, w = blockIdx.y;
+  const int b = blockIdx.x, w = g.first + blockIdx.y;
   const qsv_wblock& blk = table[blockIdx.z];  // uniform: scalar loads, no private copy
   const int tid = threadIdx.x;
   WBCheck chk;
@@ -422,7 +423,7 @@ __global__ void __launch_bounds__(kWB)
                         const T* __restrict__ dout, int64_t out_elems, double* __restrict__ drot,
                         double* __restrict__ ddamp) {
   __shared__ double F[4 * 256], G[64 * 65], W[64 * 65], dF[256];
-  const int b = blockIdx.x, w = blockIdx.y;
+  const int b = blockIdx.x, w = g.first + blockIdx.y;
   const qsv_wblock& blk = table[blockIdx.z];  // uniform: scalar loads, no private copy
   const int tid = threadIdx.x, D = wb_dim(blk.nq), ld = wb_ld(D);
   double* const X = W;
@@ -503,7 +504,8 @@ using namespace qsv;
 static int wb_geom(int batch, int n_windows, int span, int n_qubits, int layers,
                    const double* rot, const double* damp, const uint8_t* keep, const double* cz,
                    WBGeom& g) {
-  QSV_CHECK_ARG(batch >= 1 && batch <= 65535 && n_windows >= 1 && n_windows <= 65535,
+  QSV_CHECK_ARG(batch >= 1 && batch < (1 << 24) && n_windows >= 1 &&
+                    int64_t(batch) * n_windows < (int64_t(1) << 31),
                 "batch %d / windows %d out of range", batch, n_windows);
   QSV_CHECK_ARG(n_qubits >= 1 && n_qubits <= QSV_MAX_RANK, "qubits %d", n_qubits);
   QSV_CHECK_ARG(span >= 1 && layers >= int64_t(span) * n_windows,
@@ -514,6 +516,7 @@ static int wb_geom(int batch, int n_windows, int span, int n_qubits, int layers,
   g.n = n_qubits;
   g.layers = layers;
   g.span = span;
+  g.first = 0;
   g.rot = rot;
   g.damp = damp;
   g.keep = keep;
@@ -528,37 +531,50 @@ static bool wb_one(int n_pos, const qsv_wblock* table) {
   return true;
 }
 
-static int wb_run(int dtype, int n_pos, const qsv_wblock* table_host,
-                  const qsv_wblock* table_dev, const WBGeom& g, void* out, int64_t out_elems,
-                  void* stream) {
-  QSV_CHECK_ARG(table_dev && out, "null pointer argument");
-  const dim3 grid(g.batch, g.nw, n_pos);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool one = wb_one(n_pos, table_host);
-  if (dtype == QSV_F64)
-    hipLaunchKernelGGL((one ? k_window_blocks<double, true> : k_window_blocks<double, false>), grid, dim3(kWB), 0, s, table_dev, g,
-                       static_cast<double*>(out), out_elems);
-  else
-    hipLaunchKernelGGL((one ? k_window_blocks<float, true> : k_window_blocks<float, false>), grid, dim3(kWB), 0, s, table_dev, g,
-                       static_cast<float*>(out), out_elems);
-  QSV_CHECK_HIP(hipGetLastError());
+// Launches of `launch(grid, g)` over all windows: a grid's second axis holds 65535.
+template <typename F>
+static int wb_launch(WBGeom g, int n_pos, F launch) {
+  constexpr int kMost = 65535;
+  for (; g.first < g.nw; g.first += kMost) {
+    launch(dim3(g.batch, g.nw - g.first < kMost ? g.nw - g.first : kMost, n_pos), g);
+    QSV_CHECK_HIP(hipGetLastError());
+    if (g.nw - g.first <= kMost) break;
+  }
   return QSV_OK;
 }
 
-static int wb_run_backward(int dtype, int n_pos, const qsv_wblock* table_dev, const WBGeom& g,
+static int wb_run(int dtype, int n_pos, const qsv_wblock* table_host,
+                  const qsv_wblock* table_dev, const WBGeom& geom, void* out, int64_t out_elems,
+                  void* stream) {
+  QSV_CHECK_ARG(table_dev && out, "null pointer argument");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool one = wb_one(n_pos, table_host);
+  return wb_launch(geom, n_pos, [&](dim3 grid, const WBGeom& g) {
+    if (dtype == QSV_F64) {
+      const auto kern = one ? k_window_blocks<double, true> : k_window_blocks<double, false>;
+      hipLaunchKernelGGL(kern, grid, dim3(kWB), 0, s, table_dev, g, static_cast<double*>(out),
+                         out_elems);
+    } else {
+      const auto kern = one ? k_window_blocks<float, true> : k_window_blocks<float, false>;
+      hipLaunchKernelGGL(kern, grid, dim3(kWB), 0, s, table_dev, g, static_cast<float*>(out),
+                         out_elems);
+    }
+  });
+}
+
+static int wb_run_backward(int dtype, int n_pos, const qsv_wblock* table_dev, const WBGeom& geom,
                            const void* dout, int64_t out_elems, double* drot, double* ddamp_part,
                            void* stream) {
   QSV_CHECK_ARG(table_dev && dout && drot && ddamp_part, "null pointer argument");
-  const dim3 grid(g.batch, g.nw, n_pos);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == QSV_F64)
-    hipLaunchKernelGGL(k_window_blocks_bwd<double>, grid, dim3(kWB), 0, s, table_dev, g,
-                       static_cast<const double*>(dout), out_elems, drot, ddamp_part);
-  else
-    hipLaunchKernelGGL(k_window_blocks_bwd<float>, grid, dim3(kWB), 0, s, table_dev, g,
-                       static_cast<const float*>(dout), out_elems, drot, ddamp_part);
-  QSV_CHECK_HIP(hipGetLastError());
-  return QSV_OK;
+  return wb_launch(geom, n_pos, [&](dim3 grid, const WBGeom& g) {
+    if (dtype == QSV_F64)
+      hipLaunchKernelGGL(k_window_blocks_bwd<double>, grid, dim3(kWB), 0, s, table_dev, g,
+                         static_cast<const double*>(dout), out_elems, drot, ddamp_part);
+    else
+      hipLaunchKernelGGL(k_window_blocks_bwd<float>, grid, dim3(kWB), 0, s, table_dev, g,
+                         static_cast<const float*>(dout), out_elems, drot, ddamp_part);
+  });
 }
 
 extern "C" int qsv_put(const void* host, int64_t bytes, void* dst, void* stream) {
