@@ -854,6 +854,14 @@ extern "C" int qsv_circuit_blocks_count(const void* blocks) {
   return int(static_cast<const FusedBlocks*>(blocks)->blocks.size());
 }
 
+extern "C" int qsv_circuit_block_sizes(const void* blocks, int32_t* counts) {
+  const FusedBlocks* f = static_cast<const FusedBlocks*>(blocks);
+  QSV_CHECK_ARG(f && counts, "null pointer argument");
+  std::fill(counts, counts + kSlabMaxQubits + 1, 0);
+  for (const FusedBlock& b : f->blocks) ++counts[bits_of(b.q)];
+  return QSV_OK;
+}
+
 extern "C" int qsv_circuit_block_qubits(const void* blocks, int index, int32_t* qubits) {
   const FusedBlocks* f = static_cast<const FusedBlocks*>(blocks);
   QSV_CHECK_ARG(f && qubits && index >= 0 && index < int(f->blocks.size()), "no block %d", index);
@@ -908,6 +916,10 @@ extern "C" void qsv_circuit_destroy(void* plan) { delete static_cast<SlabPlan*>(
 
 extern "C" int qsv_circuit_passes(const void* plan) {
   return int(static_cast<const SlabPlan*>(plan)->passes.size());
+}
+
+extern "C" int qsv_circuit_gates(const void* plan) {
+  return int(static_cast<const SlabPlan*>(plan)->gates.size());
 }
 
 extern "C" int64_t qsv_circuit_table_bytes(const void* plan) {

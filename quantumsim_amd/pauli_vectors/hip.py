@@ -378,11 +378,12 @@ class PauliVectorHIP(PauliVectorBase):
         self._swap_in(out, extent, new_shape, new_str)
         self._used_here(self._store, self._spare)
 
-    def run_passes(self, ks, targets, ptms):
+    def run_passes(self, ks, targets, ptms, worth=None):
         """Apply a circuit of 1- and 2-qubit gates (fusion.CircuitPasses'
         arrays) in passes of several gates each; False, with nothing done,
-        on float32 vectors, under graph capture and where the layout has no
-        such passes (see fusion.apply_circuit)."""
+        on float32 vectors, under graph capture, where the layout has no
+        such passes and where ``worth(plan)`` is false (see
+        fusion.apply_circuit)."""
         from ..fusion import CircuitPasses
         if self._dtype != torch.float64 or self._store.data_ptr() % 16 or \
                 torch.cuda.is_current_stream_capturing():
@@ -390,6 +391,8 @@ class PauliVectorHIP(PauliVectorBase):
         try:
             plan = CircuitPasses(len(self._shape), self._pstr, ks, targets, ptms)
         except NotImplementedError:
+            return False
+        if worth is not None and not worth(plan):
             return False
         extent = self._data.numel()
         out = self._take_spare(extent)

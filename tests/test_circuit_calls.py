@@ -111,3 +111,37 @@ def test_replay_of_padded_layouts(n, pad_from):
         ref = _apply(x, gates)
         assert np.linalg.norm(view - ref) <= 32 * len(gates) * 2.0 ** -53 * np.linalg.norm(x)
         assert np.isnan(phys).sum() == extent - x.size
+
+
+def _pairs(kind, n, count):
+    m = n // 2
+    pairs = {'triples': [(0, 1), (m, m + 1), (1, 2), (m + 1, m + 2)],
+             'chain of triples': [t for b in range(0, n - 2, 3) for t in ((b, b + 1), (b + 1, b + 2))],
+             'brick': [(q, q + 1) for p in (0, 1) for q in range(p, n - 1, 2)]}[kind]
+    return [pairs[i % len(pairs)] for i in range(count)]
+
+
+# ms a call on float64 vectors, in passes and in blocks of up to three qubits (14 and
+# 15 qubits: 2 and 8 GB; 11 qubits: 32 MB)
+@pytest.mark.parametrize('kind,n,count,passes_ms,blocks_ms', [
+    ('triples', 14, 24, 4.19, 1.89), ('triples', 14, 200, 31.2, 2.94),
+    ('triples', 15, 64, 40.2, 7.31), ('chain of triples', 15, 80, 50.8, 18.0),
+    ('chain of triples', 14, 200, 31.2, 4.23), ('brick', 14, 60, 13.0, 28.2),
+    ('brick', 15, 60, 57.1, 112.0), ('brick', 13, 60, 3.70, 7.49),
+    ('triples', 11, 200, 1.07, 2.13), ('triples', 9, 64, 0.33, 0.74),
+    ('triples', 13, 200, 8.24, 2.33), ('chain of triples', 9, 200, 0.85, 2.18)])
+def test_many_gates_in_few_blocks_stay_blocks(monkeypatch, kind, n, count, passes_ms, blocks_ms):
+    """A pass pays for every two-qubit gate, a dense block only once."""
+    monkeypatch.setattr(fusion, '_native_circuit', lambda pv, gates: _qubit_gates(gates, pv.n_qubits))
+    rng = np.random.default_rng(0)
+    ptm = rng.standard_normal((4,) * 4)
+
+    class Vector(_Recorder):
+        def run_passes(self, ks, targets, ptms, worth=None):
+            plan = CircuitPasses(n, [4 ** (n - 1 - q) for q in range(n)], ks, targets, ptms)
+            self.taken = worth is None or worth(plan)
+            return self.taken
+    pv = Vector(n)
+    fusion.apply_circuit(pv, [(ptm, t) for t in _pairs(kind, n, count)], 3)
+    assert pv.taken == (passes_ms < blocks_ms)
+    assert bool(pv.applied) != pv.taken
