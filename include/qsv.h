@@ -342,6 +342,10 @@ int qsv_emulate_gate_params(int batch, int layers, int own, int n, const double*
 int64_t qsv_ptm_grad_workspace_bytes(int batch, int rank, const int64_t* dims, int k,
                                      const int32_t* targets, const int32_t* dims_out_t);
 
+/* Workgroups per state that qsv_ptm_grad takes by itself (without a tile). */
+int qsv_ptm_grad_blocks(int dtype, int batch, int rank, const int64_t* dims, int k,
+                        const int32_t* targets, const int32_t* dims_out_t);
+
 /* Gradient of a PTM application with respect to the PTM, for `batch` states
  * back to back (the layout of qsv_apply_ptm_batched), PTMs up to 256
  * entries a side and 8192 entries (MFMA kernels up to 64 x 64, a float64

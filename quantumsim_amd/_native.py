@@ -76,6 +76,8 @@ _SIGNATURES = {
     'qsv_apply_ptm_batched': (ctypes.c_int, [ctypes.c_int, _vp, _vp, ctypes.c_int, ctypes.c_int,
                                              _c_i64p, ctypes.c_int, _c_i32p, _c_i32p, _vp,
                                              ctypes.c_int64, _vp]),
+    'qsv_ptm_grad_blocks': (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _c_i64p,
+                                           ctypes.c_int, _c_i32p, _c_i32p]),
     'qsv_ptm_grad_workspace_bytes': (ctypes.c_int64, [ctypes.c_int, ctypes.c_int, _c_i64p,
                                                       ctypes.c_int, _c_i32p, _c_i32p]),
     'qsv_ptm_grad': (ctypes.c_int, [ctypes.c_int, _vp, _vp, ctypes.c_int, ctypes.c_int, _c_i64p,

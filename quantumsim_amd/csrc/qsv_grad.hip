@@ -1486,12 +1486,15 @@ static int make_grad_plan(int elem_bytes, int rank, const int64_t* dims, int k,
 // round of loads a wave.  A block of 1024 is sixteen rounds, each a trip to
 // memory: six 10-qubit float32 states 35 -> 22 us for a 16 x 16 PTM, one of 11
 // qubits 71 -> 20, one qubit's 83 -> 28.
+// Not two per state in float64: 512 states of 7 qubits took 34.8 us on two, 28.5 on one
+// (three, 340 states: 20.7 against 23.6; float32 on two 18.1 against 25.3).
 constexpr uint32_t kGradFill = 1024;
-static int grad_blocks(uint32_t n_orbits, int batch) {
+static int grad_blocks(uint32_t n_orbits, int batch, bool f64) {
   const uint32_t B = uint32_t(std::max(batch, 1));
   uint32_t b = (n_orbits + 1023) / 1024;
   b = std::min(b, (4096 + B - 1) / B);
-  b = std::max(b, std::min((n_orbits + 63) / 64, kGradFill / B));
+  const uint32_t fill = kGradFill / B;
+  if (!(f64 && fill == 2)) b = std::max(b, std::min((n_orbits + 63) / 64, fill));
   return int(b < 1 ? 1 : (b > kGradBlocks ? kGradBlocks : b));
 }
 
@@ -1521,10 +1524,10 @@ static int max_grad_blocks(const GradPlan& p) {
   return p.big ? kGradBigBlocks : (grad_wide(p) ? kGrad64Blocks : kGradBlocks);
 }
 
-static int default_grad_blocks(const GradPlan& p, int batch) {
+static int default_grad_blocks(const GradPlan& p, int batch, bool f64) {
   return p.big ? grad_big_blocks(p.n_orbits, batch)
                : (grad_wide(p) ? grad64_blocks(p.n_orbits, batch)
-                               : grad_blocks(p.n_orbits, batch));
+                               : grad_blocks(p.n_orbits, batch, f64));
 }
 
 // Fused backward of a dense 64 x 64 block of float64 states (float32 runs
@@ -1741,6 +1744,15 @@ extern "C" int64_t qsv_batched_backward_workspace_bytes(int dtype, int batch, in
   return dtype == QSV_F32 && least > 0 ? std::max<int64_t>(least, kBwdBlocks * 64 * 64 * 8) : least;
 }
 
+extern "C" int qsv_ptm_grad_blocks(int dtype, int batch, int rank, const int64_t* dims, int k,
+                                   const int32_t* targets, const int32_t* dims_out_t) {
+  QSV_CHECK_ARG(dtype == QSV_F32 || dtype == QSV_F64, "unknown dtype %d", dtype);
+  QSV_CHECK_ARG(batch >= 1 && batch <= 65535, "batch %d outside [1, 65535]", batch);
+  GradPlan p;
+  const int rc = make_grad_plan(dtype_size(dtype), rank, dims, k, targets, dims_out_t, p);
+  return rc ? rc : default_grad_blocks(p, batch, dtype == QSV_F64);
+}
+
 template <typename T>
 static void launch_grad(const GradPlan& p, int vn, bool quad, dim3 grid, const void* x,
                         const void* ybar, double* partial, hipStream_t s) {
@@ -1816,7 +1828,8 @@ static int ptm_grad_run(int dtype, const void* x, const void* ybar, int batch, i
   QSV_CHECK_ARG(!tile || tile->grad_blocks <= max_grad_blocks(p),
                 "tile: grad_blocks %d above %d for a %d x %d PTM", tile ? tile->grad_blocks : 0,
                 max_grad_blocks(p), p.dout, p.din);
-  int nb = tile && tile->grad_blocks > 0 ? tile->grad_blocks : default_grad_blocks(p, batch);
+  int nb = tile && tile->grad_blocks > 0 ? tile->grad_blocks
+                                         : default_grad_blocks(p, batch, dtype == QSV_F64);
   const int64_t per_block = int64_t(batch) * p.din * p.dout * 8;
   if (shrink) {
     QSV_CHECK_ARG(per_block <= partial_bytes,
@@ -2415,7 +2428,7 @@ extern "C" int qsv_emulate_ptm_grad(int dtype, const double* x, const double* yb
                                                  : grad64_blocks(p.n_orbits, 1),
                           dptm, p.quad ? kGrad64UnrollQuad : kGrad64Unroll);
   const int VN = p.vn, waves = kBlock / 64;
-  const int nb = grad_blocks_forced > 0 ? grad_blocks_forced : grad_blocks(p.n_orbits, 1);
+  const int nb = grad_blocks_forced > 0 ? grad_blocks_forced : grad_blocks(p.n_orbits, 1, dtype == QSV_F64);
   if (vn_out) *vn_out = VN;
   const uint32_t STEP = 4 * VN, nsteps = (p.n_orbits + STEP - 1) / STEP;
   std::vector<int> used(p.n_orbits, 0);
