@@ -534,7 +534,10 @@ def run_schedule(x0, steps, targets, segments, shape, checkpoint_every=1):
             raise ValueError('segments must start with all {} states and hand each '
                              'segment the previous one\'s continuing states'.format(B))
         prev = cont
-        gs = np.ascontiguousarray(np.array(gates, dtype=np.int32).reshape(-1, 2))
+        try:
+            gs = np.array(gates, dtype=np.int64).reshape(-1, 2)
+        except OverflowError:
+            raise ValueError('a gate outside the steps tensors') from None
         bad = (gs < 0).any(1) | (gs[:, 0] >= len(steps))
         if not bad.any():
             bad = gs[:, 1] >= n_steps[gs[:, 0]]
@@ -542,7 +545,8 @@ def run_schedule(x0, steps, targets, segments, shape, checkpoint_every=1):
             raise ValueError('gate ({}, {}) outside the steps tensors'.format(
                 *gs[int(np.argmax(bad))]))
         seen.append(gs[:, 0] * np.int64(total + 1) + gs[:, 1])
-        parts.append((int(active), int(cont), gs, np.unique(gs[:, 0]).tolist()))
+        parts.append((int(active), int(cont), np.ascontiguousarray(gs, dtype=np.int32),
+                      np.unique(gs[:, 0]).tolist()))
     if seen and np.unique(np.concatenate(seen)).size != sum(len(s) for s in seen):
         raise ValueError('each (position, step) PTM drives one gate')
     if prev != 0:
