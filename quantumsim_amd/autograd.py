@@ -535,9 +535,13 @@ def run_schedule(x0, steps, targets, segments, shape, checkpoint_every=1):
                              'segment the previous one\'s continuing states'.format(B))
         prev = cont
         try:
-            gs = np.array(gates, dtype=np.int64).reshape(-1, 2)
+            gs = np.array(gates, dtype=np.int64)
         except OverflowError:
             raise ValueError('a gate outside the steps tensors') from None
+        if gs.size == 0:
+            gs = gs.reshape(0, 2)
+        elif gs.ndim != 2 or gs.shape[1] != 2:
+            raise ValueError('gates are pairs (position, step)')
         bad = (gs < 0).any(1) | (gs[:, 0] >= len(steps))
         if not bad.any():
             bad = gs[:, 1] >= n_steps[gs[:, 0]]

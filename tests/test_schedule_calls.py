@@ -17,3 +17,13 @@ def test_gates_beyond_the_steps_are_refused(gate):
     steps = [torch.zeros((3, 2, 4, 4))]
     with pytest.raises(ValueError, match='outside the steps'):
         run_schedule(x0, steps, [(0,)], [(2, 0, [(0, 0), gate])], (4, 4))
+
+
+@pytest.mark.parametrize('gates', [[(0, 0, 1), (0, 1, 2)], [(0,), (1,)], [0, 0, 0, 1],
+                                   [(0, 0), (0,)]])
+def test_gates_that_are_no_pairs_are_refused(gates):
+    """Six numbers are not three gates."""
+    x0 = torch.zeros((2, 16))
+    steps = [torch.zeros((3, 2, 4, 4))] * 3
+    with pytest.raises((TypeError, ValueError)):
+        run_schedule(x0, steps, [(0,)] * 3, [(2, 0, gates)], (4, 4))
