@@ -80,8 +80,9 @@ struct Segment {
     if (finals.n == kGradFinals || ws_used + most > ws_bytes)
       if (const int rc = sums()) return rc;
     return launch(kind, p, [&] {
+      const int before = finals.n;
       const int rc = f(ws + ws_used, most < ws_bytes - ws_used ? most : ws_bytes - ws_used);
-      if (rc) return rc;
+      if (rc || finals.n == before) return rc;  // no states: no partials
       const GradFinal& l = finals.it[finals.n - 1];
       ws_used += (int64_t(l.nb) * l.dd * active * 8 + 255) / 256 * 256;
       return hook ? sums() : int(QSV_OK);  // a counted launch has its sum with it

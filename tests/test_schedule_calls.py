@@ -27,3 +27,27 @@ def test_gates_that_are_no_pairs_are_refused(gates):
     steps = [torch.zeros((3, 2, 4, 4))] * 3
     with pytest.raises((TypeError, ValueError)):
         run_schedule(x0, steps, [(0,)] * 3, [(2, 0, gates)], (4, 4))
+
+
+@pytest.mark.parametrize('dtype', [nat.QSV_F32, nat.QSV_F64])
+@pytest.mark.parametrize('fused', [0, 1])
+def test_no_running_state(dtype, fused):
+    """Segments without states launch nothing, gradients included; the adjoint's
+    buffers change places gate by gate all the same."""
+    L, n = nat.lib(), 7
+    dims = nat.i64([4] * n)
+    rows = (nat.SchedPos * 1)()
+    r = rows[0]
+    r.k, r.n_steps, r.fused, r.targets[:3] = 3, 3, fused, (1, 2, 4)
+    r.ptm = r.ptm_t = r.grad_ptm = 4096
+    r.step, r.state, r.workspace = 64 * 64, 64 * 64, 0
+    gates = np.array([(0, 0), (0, 1), (0, 2)], dtype=np.int32)
+    ptrs = (ctypes.c_void_p * 3)(4096, 4096, 8192)
+    assert L.qsv_schedule_forward(dtype, n, dims, 1, rows, 0, 3, gates.ctypes.data, 4096, ptrs,
+                                  nat.SchedHook(), None) == 0
+    for every in (1, 2, 3):
+        cur = ctypes.c_int32(7)
+        assert L.qsv_schedule_backward(dtype, n, dims, 1, rows, 0, 3, gates.ctypes.data, every,
+                                       ptrs, ptrs, ptrs, 0, 4096, 0, ctypes.byref(cur),
+                                       nat.SchedHook(), None) == 0
+        assert cur.value == 1
