@@ -371,7 +371,7 @@ class _SchedulePositions:
     def hook(self):
         """Counts every launch in the ledger in force, if any."""
         led = _ledger.active()
-        if led is None:
+        if led is None or not self.steps:
             return nat.SchedHook()
         N, es = math.prod(self.shape), self.steps[0].element_size()
         events = []

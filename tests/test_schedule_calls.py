@@ -51,3 +51,12 @@ def test_no_running_state(dtype, fused):
                                        ptrs, ptrs, ptrs, 0, 4096, 0, ctypes.byref(cur),
                                        nat.SchedHook(), None) == 0
         assert cur.value == 1
+
+
+def test_schedule_without_positions_under_a_ledger():
+    from quantumsim_amd.ledger import Ledger
+    x0 = torch.ones((2, 16), requires_grad=True)
+    with Ledger(timed=False):
+        out = run_schedule(x0, [], [], [(2, 1, []), (1, 0, [])], (4, 4))
+        gx, = torch.autograd.grad(out.sum(), [x0])
+    assert torch.equal(out, x0) and torch.equal(gx, torch.ones_like(x0))
