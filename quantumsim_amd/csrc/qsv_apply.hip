@@ -822,13 +822,9 @@ static bool fits_inline(int64_t din, int64_t dout) {
   return din <= kInline && dout <= kInline;
 }
 
-// bytes of the device table for a PTM of dout x din (0 when inline)
-static int64_t table_bytes(int dtype, int64_t din, int64_t dout, bool with_ptm) {
-  if (fits_inline(din, dout)) return 0;
-  const int64_t dinp = round_up(din, 16), doutp = round_up(dout, 16);
-  int64_t b = (dinp + doutp) * 8;
-  if (with_ptm) b += dinp * doutp * dtype_size(dtype);
-  return round_up(b, 256);
+// bytes of the device copy of a host PTM of dout x din (0 when inline)
+static int64_t table_bytes(int dtype, int64_t din, int64_t dout) {
+  return fits_inline(din, dout) ? 0 : round_up(din * dout * dtype_size(dtype), 256);
 }
 
 static bool use_fused(const Plan& p) {
@@ -969,7 +965,7 @@ extern "C" int64_t qsv_apply_ptm_workspace_bytes(int dtype, int k, const int32_t
     din *= dims_in_t[j];
     dout *= dims_out_t[j];
   }
-  return table_bytes(dtype, din, dout, true);
+  return table_bytes(dtype, din, dout);
 }
 
 extern "C" int qsv_apply_ptm(int dtype, const void* in, void* out, int rank,
@@ -999,7 +995,7 @@ extern "C" int qsv_apply_ptm_strided(int dtype, const void* in, void* out, int r
     return small ? run_inline<float, 4>(p, ptm_f64, in, out, s)
                  : run_inline<float, 16>(p, ptm_f64, in, out, s);
   }
-  const int64_t need = table_bytes(dtype, p.din, p.dout, true);
+  const int64_t need = table_bytes(dtype, p.din, p.dout);
   QSV_CHECK_ARG(workspace && workspace_bytes >= need,
                 "a %d x %d PTM needs a workspace of %lld bytes", p.dout, p.din,
                 (long long)need);

@@ -1006,6 +1006,7 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// Resident blocks of `kernel` over the device (occupancy x CUs).
 static uint32_t resident_blocks(const void* kernel) {
   int dev = 0, cus = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -1064,9 +1065,6 @@ __global__ void __launch_bounds__(kBlock)
   lds_barrier();
   dir_apply<true>(st, pb, lane, g, t, yo, y);
 }
-
-// Resident blocks of `kernel` over the device (occupancy x CUs).
-static uint32_t resident_blocks(const void* kernel);
 
 static uint32_t apply64d_cap() {
   static const uint32_t cap =
