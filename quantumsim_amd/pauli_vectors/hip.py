@@ -369,14 +369,16 @@ class PauliVectorHIP(PauliVectorBase):
         L = nat.lib()
         apply, data = ((L.qsv_apply_ptm_dev_strided, ptm.data_ptr()) if on_device else
                        (L.qsv_apply_ptm_strided, ptm.__array_interface__['data'][0]))
+        raw = _raw_stream(self._device)
         rc = apply(code, self._store.data_ptr(), out.data_ptr(), len(shape), in_dims, in_str,
                    out_str, k, _i32s(qubits), _i32s(dims_out_t), data, ws, ws_bytes,
-                   _stream(self._device))
+                   ctypes_void(raw))
         if rc != 0:
             self._spare = out
             nat.check(rc, 'apply_ptm')
         self._swap_in(out, extent, new_shape, new_str)
-        self._used_here(self._store, self._spare)
+        if not self._store_home == self._spare_home == raw:
+            self._used_here(self._store, self._spare)
 
     def run_passes(self, ks, targets, ptms, worth=None):
         """Apply a circuit of 1- and 2-qubit gates (fusion.CircuitPasses'
