@@ -947,6 +947,8 @@ extern "C" int qsv_circuit_run(const void* plan, const void* in, void* out, cons
   double* dst = static_cast<double*>(out);
   const SlabGate* gates = static_cast<const SlabGate*>(table_dev);
   const bool big = 2 * p->extent * 8 > nt_threshold_bytes();
+  if (p->passes.empty() && in != out)  // no gates
+    QSV_CHECK_HIP(hipMemcpyAsync(out, in, p->extent * 8, hipMemcpyDeviceToDevice, s));
   for (const SlabPass& ps : p->passes) {
     // nontemporal only on whole lines, as in the other kernels
     const bool nt = big && ps.run128;

@@ -145,3 +145,17 @@ def test_many_gates_in_few_blocks_stay_blocks(monkeypatch, kind, n, count, passe
     fusion.apply_circuit(pv, [(ptm, t) for t in _pairs(kind, n, count)], 3)
     assert pv.taken == (passes_ms < blocks_ms)
     assert bool(pv.applied) != pv.taken
+
+
+@pytest.mark.gpu
+def test_circuit_without_gates_copies():
+    import torch
+    n = 3
+    empty = np.zeros(0, dtype=np.int32)
+    plan = CircuitPasses(n, [16, 4, 1], empty, empty, np.zeros(0))
+    assert plan.passes == 0
+    x = torch.randn(64, dtype=torch.float64, device='cuda')
+    y = torch.zeros_like(x)
+    plan.run(x.data_ptr(), y.data_ptr(), None, torch.cuda.current_stream().cuda_stream or None)
+    torch.cuda.synchronize()
+    assert torch.equal(x, y)
