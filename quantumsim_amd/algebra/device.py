@@ -71,9 +71,10 @@ def _apply(x, dims, target, M):
     tg, do = nat.i32([target, n]), nat.i32([mo, 2])
     ws = nat.check(L.qsv_apply_ptm_workspace_bytes(nat.QSV_F64, 2, nat.i32([dims[target], 2]), do),
                    'apply_ptm')
-    buf = _Scratch.get(x.device, 'ptm', ws).data_ptr() if ws else None
+    buf = _Scratch.get(x.device, 'ptm', ws) if ws else None
     rc = L.qsv_apply_ptm(nat.QSV_F64, x.data_ptr(), y.data_ptr(), n + 1, nat.i64(full), 2, tg, do,
-                         P.ctypes.data_as(nat._c_f64p), buf, ws, _stream(x.device))
+                         P.ctypes.data_as(nat._c_f64p), None if buf is None else buf.data_ptr(), ws,
+                         _stream(x.device))
     nat.check(rc, 'apply_ptm')
     return y, out_dims
 

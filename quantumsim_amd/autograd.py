@@ -43,13 +43,16 @@ def _stream():
 class _Workspace:
     """Scratch of the PTM-gradient partial sums, one buffer per (device,
     stream): launches on one stream run in order and may share it, launches
-    on two streams may overlap and must not.  Grown outside graph capture
-    (the eager warm-up sizes it)."""
+    on two streams may overlap and must not.  Under graph capture a buffer of
+    the graph's own pool: a graph that held this one's address would write to
+    memory given back as soon as a larger one replaces it."""
     _bufs = {}
 
     @classmethod
     def get(cls, device, nbytes, use=None):
         """``use``: a purpose with a buffer of its own."""
+        if torch.cuda.is_current_stream_capturing():
+            return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
         key = (device, torch.cuda.current_stream(device).cuda_stream, use)
         t = cls._bufs.get(key)
         if t is None or t.numel() < nbytes:
@@ -288,8 +291,8 @@ def capture_step(fn, warmup=1, stream=None):
     """Record one call of ``fn`` (a forward + backward built from this
     module's operations and torch ops, with no host synchronisation) in a
     HIP graph.  ``fn`` runs ``warmup`` times eagerly on ``stream`` first (a
-    new stream of default priority if None), which sizes every buffer and
-    scratch area, then the eager blocks are handed back and the call is
+    new stream of default priority if None), which builds every shared
+    constant, then the eager blocks are handed back and the call is
     captured.  Returns (graph, stream, outputs): ``graph.replay()`` on
     ``stream`` recomputes ``outputs`` in place."""
     if stream is None:
@@ -317,8 +320,7 @@ def run_circuit(x0, gates, shape, checkpoint_every=8):
 
 # Partial sums of a schedule's PTM gradients kept per stream: sixteen gates of
 # six 8-qubit circuits (25 MB) or five of six 11-qubit ones, and the partials are
-# still in the 256 MB last-level cache when they are summed.  A fixed size, so that
-# the buffer a captured graph holds is replaced only for a larger single gate.
+# still in the 256 MB last-level cache when they are summed.
 _SCHEDULE_SCRATCH = 64 << 20
 
 

@@ -86,12 +86,15 @@ class _Scratch:
     Calls on one stream use a buffer in stream order; calls issued on
     different streams get different buffers, so they cannot overwrite a
     table another stream's kernel is still reading, and a buffer that grows
-    is handed back to the allocator on the stream it was used on."""
+    is handed back to the allocator on the stream it was used on.  A captured
+    launch, which keeps its buffer's address, gets one of the graph's pool."""
 
     _bufs = {}
 
     @classmethod
     def get(cls, device, purpose, nbytes):
+        if torch.cuda.is_current_stream_capturing():
+            return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
         key = (device, _raw_stream(device), purpose)
         t = cls._bufs.get(key)
         if t is None or t.numel() < nbytes:
@@ -365,14 +368,14 @@ class PauliVectorHIP(PauliVectorBase):
         out = self._take_spare(extent)
         code = self._code()
         ws_bytes = _ptm_workspace(code, dims_in_t, dims_out_t)
-        ws = _Scratch.get(self._device, 'ptm', ws_bytes).data_ptr() if ws_bytes else None
+        ws = _Scratch.get(self._device, 'ptm', ws_bytes) if ws_bytes else None
         L = nat.lib()
         apply, data = ((L.qsv_apply_ptm_dev_strided, ptm.data_ptr()) if on_device else
                        (L.qsv_apply_ptm_strided, ptm.__array_interface__['data'][0]))
         raw = _raw_stream(self._device)
         rc = apply(code, self._store.data_ptr(), out.data_ptr(), len(shape), in_dims, in_str,
-                   out_str, k, _i32s(qubits), _i32s(dims_out_t), data, ws, ws_bytes,
-                   ctypes_void(raw))
+                   out_str, k, _i32s(qubits), _i32s(dims_out_t), data,
+                   None if ws is None else ws.data_ptr(), ws_bytes, ctypes_void(raw))
         if rc != 0:
             self._spare = out
             nat.check(rc, 'apply_ptm')
@@ -457,10 +460,11 @@ class PauliVectorHIP(PauliVectorBase):
             ws_bytes = L.qsv_apply_ptm_workspace_bytes(
                 nat.QSV_F64, 1, nat.i32([tr.shape[1]]), nat.i32([tr.shape[0]]))
             nat.check(ws_bytes, 'diagonal')
-            ws = _Scratch.get(self._device, 'ptm', ws_bytes).data_ptr() if ws_bytes else None
+            ws = _Scratch.get(self._device, 'ptm', ws_bytes) if ws_bytes else None
             rc = L.qsv_apply_ptm(nat.QSV_F64, cur.data_ptr(), nxt.data_ptr(), rank,
                                  nat.i64(dims), 1, nat.i32([q]), nat.i32([tr.shape[0]]),
-                                 tr.ctypes.data_as(nat._c_f64p), ws, ws_bytes, s)
+                                 tr.ctypes.data_as(nat._c_f64p),
+                                 None if ws is None else ws.data_ptr(), ws_bytes, s)
             nat.check(rc, 'diagonal')
             cur, dims = nxt[:math.prod(nxt_dims)], nxt_dims
         return cur.view(tuple(plan.dims_hilbert))
@@ -553,12 +557,12 @@ class PauliVectorHIP(PauliVectorBase):
                               device=self._device)
             ws_bytes = nat.check(L.qsv_apply_ptm_workspace_bytes(
                 code, 1, nat.i32([shape[q]]), nat.i32([1])), 'partial_trace')
-            ws = _Scratch.get(self._device, 'ptm', ws_bytes).data_ptr() if ws_bytes else None
+            ws = _Scratch.get(self._device, 'ptm', ws_bytes) if ws_bytes else None
             rc = L.qsv_apply_ptm_strided(
                 code, cur.data_ptr(), nxt.data_ptr(), len(shape), nat.i64(shape),
                 nat.i64(strides) if strides is not None else None, None, 1, nat.i32([q]),
-                nat.i32([1]), np.ascontiguousarray(t).ctypes.data_as(nat._c_f64p), ws,
-                ws_bytes, s)
+                nat.i32([1]), np.ascontiguousarray(t).ctypes.data_as(nat._c_f64p),
+                None if ws is None else ws.data_ptr(), ws_bytes, s)
             nat.check(rc, 'partial_trace')
             self._used_here(cur)
             cur, shape, strides = nxt[:math.prod(new_shape)], new_shape, None
