@@ -1,6 +1,6 @@
 // The launches of a batched gate schedule, issued from one call per segment.
 //
-// A batch of 8-11-qubit circuits makes about 1900 launches a training step, each
+// A batch of 8-11-qubit circuits makes about 1650 launches a training step, each
 // of 10-50 us on the device; issued one library call at a time from the
 // interpreter they cost 13 us each on the host (allocation, views, argument
 // arrays), 28 of the step's 32 ms, with the device idle between them.  The same
