@@ -216,24 +216,24 @@ int qsv_circuits_forward(int dtype, int n_circuits, const qsv_circuit* circs_dev
  *                        passes cannot read in aligned runs (the innermost
  *                        axis not of stride 1 among them).
  *   qsv_circuit_passes   number of passes
- *   qsv_circuit_gates    number of two-qubit blocks in all passes
  *   qsv_circuit_table    writes the blocks' tables (qsv_circuit_table_bytes)
  *                        to host memory; the caller copies them to the device
  *   qsv_circuit_run      launches the passes: in -> out, the later ones in
  *                        place on out (in is only read; both may be the same)
  * The same gates fused into dense blocks of up to max_qudits qubits (the
  * blocks and order of quantumsim_amd.fusion.fuse):
- *   qsv_circuit_blocks_create  plans them; freed with qsv_circuit_blocks_destroy
+ *   qsv_circuit_blocks_create  plans them; freed with qsv_circuit_blocks_destroy;
+ *                              QSV_ENOTSUP: PTM entries that are not finite
  *   qsv_circuit_blocks_count   their number
- *   qsv_circuit_block_sizes    counts[k]: those of k qubits, k = 0..16
  *   qsv_circuit_block_qubits   a block's qubits, ascending; returns how many
- *   qsv_circuit_block_ptm      its row-major 4^k x 4^k PTM */
+ *   qsv_circuit_block_ptm      its row-major 4^k x 4^k PTM
+ *   qsv_circuit_pays           1 if the passes are estimated to take no longer
+ *                              than the blocks of the same circuit, else 0 */
 int qsv_circuit_create(int n_qubits, const int64_t* strides, int n_gates, const int32_t* ks,
                        const int32_t* targets, const double* ptms,
                        void** plan_out);
 void qsv_circuit_destroy(void* plan);
 int qsv_circuit_passes(const void* plan);
-int qsv_circuit_gates(const void* plan);
 int64_t qsv_circuit_table_bytes(const void* plan);
 int qsv_circuit_table(const void* plan, void* host);
 int qsv_circuit_run(const void* plan, const void* in, void* out, const void* table_dev,
@@ -243,7 +243,7 @@ int qsv_circuit_blocks_create(int n_qubits, int n_gates, const int32_t* ks,
                               void** blocks_out);
 void qsv_circuit_blocks_destroy(void* blocks);
 int qsv_circuit_blocks_count(const void* blocks);
-int qsv_circuit_block_sizes(const void* blocks, int32_t* counts);
+int qsv_circuit_pays(const void* plan, const void* blocks);
 int qsv_circuit_block_qubits(const void* blocks, int index, int32_t* qubits);
 int qsv_circuit_block_ptm(const void* blocks, int index, double* ptm);
 /* CPU replay of the passes on v (float64, the plan's layout), every access

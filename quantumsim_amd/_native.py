@@ -155,7 +155,6 @@ _SIGNATURES = {
                                           _c_i32p, _c_f64p, ctypes.POINTER(_vp)]),
     'qsv_circuit_destroy': (None, [_vp]),
     'qsv_circuit_passes': (ctypes.c_int, [_vp]),
-    'qsv_circuit_gates': (ctypes.c_int, [_vp]),
     'qsv_circuit_table_bytes': (ctypes.c_int64, [_vp]),
     'qsv_circuit_table': (ctypes.c_int, [_vp, _vp]),
     'qsv_circuit_run': (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp]),
@@ -163,7 +162,7 @@ _SIGNATURES = {
                                                  _c_f64p, ctypes.c_int, ctypes.POINTER(_vp)]),
     'qsv_circuit_blocks_destroy': (None, [_vp]),
     'qsv_circuit_blocks_count': (ctypes.c_int, [_vp]),
-    'qsv_circuit_block_sizes': (ctypes.c_int, [_vp, _c_i32p]),
+    'qsv_circuit_pays': (ctypes.c_int, [_vp, _vp]),
     'qsv_circuit_block_qubits': (ctypes.c_int, [_vp, ctypes.c_int, _c_i32p]),
     'qsv_circuit_block_ptm': (ctypes.c_int, [_vp, ctypes.c_int, _c_f64p]),
     'qsv_emulate_circuit': (ctypes.c_int, [_vp, _c_f64p]),

@@ -232,11 +232,6 @@ class CircuitPasses:
     def passes(self):
         return self._lib.qsv_circuit_passes(self.handle)
 
-    @property
-    def gates(self):
-        """Two-qubit blocks in all passes."""
-        return self._lib.qsv_circuit_gates(self.handle)
-
     def table(self, device):
         """The blocks' tables on ``device``, copied from pinned memory on the
         current stream."""
@@ -254,7 +249,9 @@ class CircuitPasses:
 class QubitBlocks:
     """``fuse`` for the circuits ``_qubit_gates`` takes, planned and composed
     in the library: the same blocks in the same order, PTMs equal to
-    rounding.  Iterating composes one block at a time: (ptm, qubits)."""
+    rounding.  Iterating composes one block at a time: (ptm, qubits).
+    NotImplementedError for PTMs that are not finite (the library skips zeros
+    where ``fuse`` makes 0 * inf a NaN)."""
 
     def __init__(self, n, ks, targets, ptms, max_qudits):
         import ctypes
@@ -273,12 +270,10 @@ class QubitBlocks:
     def __len__(self):
         return self._lib.qsv_circuit_blocks_count(self.handle)
 
-    def sizes(self):
-        """Number of blocks of k qubits, k = 0..16."""
-        counts = np.zeros(17, dtype=np.int32)
-        nat.check(self._lib.qsv_circuit_block_sizes(
-            self.handle, counts.ctypes.data_as(nat._c_i32p)), 'fuse')
-        return counts.tolist()
+    def dearer_than(self, passes):
+        """Whether a CircuitPasses of the same gates takes no longer
+        (qsv_circuit_pays)."""
+        return bool(self._lib.qsv_circuit_pays(passes.handle, self.handle))
 
     def __iter__(self):
         qubits = np.zeros(32, dtype=np.int32)
@@ -293,8 +288,7 @@ class QubitBlocks:
 
 def _qubit_gates(gates, n):
     """(ks, targets, ptms) arrays of a circuit of 1- and 2-qubit gates with
-    real, finite square PTMs on n qubits, or None if it holds any other gate
-    (the library skips zeros where ``fuse`` makes 0 * inf a NaN)."""
+    real square PTMs on n qubits, or None if it holds any other gate."""
     ks, targets, ptms = [], [], []
     for ptm, qudits in gates:
         p = np.asarray(ptm)
@@ -307,10 +301,8 @@ def _qubit_gates(gates, n):
         ks.append(k)
         targets += q if k == 2 else (q[0], -1)
         ptms.append(p.reshape(-1))
-    flat = np.concatenate(ptms).astype(np.float64, copy=False)
-    if not np.isfinite(flat).all():
-        return None
-    return np.array(ks, dtype=np.int32), np.array(targets, dtype=np.int32), flat
+    return (np.array(ks, dtype=np.int32), np.array(targets, dtype=np.int32),
+            np.concatenate(ptms).astype(np.float64, copy=False))
 
 
 def _native_circuit(pv, gates):
@@ -325,25 +317,6 @@ def _native_circuit(pv, gates):
     return _qubit_gates(gates, n)
 
 
-def _passes_pay(n, n_gates, blocks, plan):
-    """Whether the passes of ``plan`` take no longer than ``blocks``' dense PTMs
-    on n qubits.  Milliseconds as measured: on 14 qubits (2 GB) a pass takes 0.37
-    and 0.145 for each of its two-qubit gates, at least 0.72 (its traffic); a dense
-    block 0.72, 0.75, 0.9 and 2.0 for one to four qubits; in proportion to the
-    vector otherwise.  The host spends 4 us a gate on the passes, 10.5 a gate and
-    30 a block on the blocks.  So passes on brickwork (14 qubits, 60 gates: 13.0 ms
-    against 28.2) and on small vectors, blocks where many gates meet on few qubits
-    (two triples of qubits, 200 gates: 2.9 ms against 31.2)."""
-    scale = 4.0 ** (n - 14)
-    passes = scale * max(0.72 * plan.passes, 0.37 * plan.passes + 0.145 * plan.gates) + \
-        0.004 * n_gates
-    dense = 0.0105 * n_gates
-    for k, count in enumerate(blocks.sizes()):
-        once = (0.72, 0.72, 0.75, 0.9)[k] if k < 4 else 2.0 * 4.0 ** (k - 4)
-        dense += count * (scale * once + 0.03)
-    return passes <= dense
-
-
 def apply_circuit(pv, gates, max_qudits=3):
     """Apply ``gates`` = [(ptm, qudits), ...] (PTMs in ``pv``'s bases) to the
     Pauli vector ``pv``, fused into blocks of up to ``max_qudits`` qudits
@@ -354,22 +327,30 @@ def apply_circuit(pv, gates, max_qudits=3):
     (csrc/qsv_slab.hip): the same product, rounded in another order.  Float32
     vectors keep the blocks, whose rounding the populations of a float32 run
     carry to their last digit; so do circuits of one block (one pass either
-    way) or of few blocks of many gates (_passes_pay), layouts without aligned
-    runs and graph capture (the passes' tables are copied from host memory).
-    Any other circuit is fused by ``fuse``."""
+    way) or of few blocks of many gates (QubitBlocks.dearer_than), layouts
+    without aligned runs and graph capture (the passes' tables are copied from
+    host memory).  Any other circuit is fused by ``fuse``."""
     if max_qudits is None or max_qudits <= 1:
         for ptm, qudits in gates:
             pv.apply_ptm(np.asarray(ptm), *qudits)
         return len(gates)
-    gates = [(ptm, tuple(qudits)) for ptm, qudits in gates]
-    arrays = _native_circuit(pv, gates) if gates else None
-    if arrays is None:
+    gates = list(gates)
+    try:
+        arrays = _native_circuit(pv, gates) if gates else None
+    except TypeError:                # targets without a length: read once each
+        gates = [(ptm, tuple(qudits)) for ptm, qudits in gates]
+        arrays = _native_circuit(pv, gates)
+    fused = None
+    if arrays is not None:
+        try:
+            fused = QubitBlocks(pv.n_qubits, *arrays, min(max_qudits, pv.n_qubits))
+        except NotImplementedError:
+            pass
+        else:
+            if len(fused) > 1 and pv.run_passes(*arrays, fused.dearer_than):
+                return len(fused)
+    if fused is None:
         fused = fuse(gates, list(pv.dim_pauli), max_qudits)
-    else:
-        fused = QubitBlocks(pv.n_qubits, *arrays, min(max_qudits, pv.n_qubits))
-        if len(fused) > 1 and pv.run_passes(
-                *arrays, lambda plan: _passes_pay(pv.n_qubits, len(gates), fused, plan)):
-            return len(fused)
     for ptm, qudits in fused:
         pv.apply_ptm(ptm, *qudits)
     return len(fused)
