@@ -307,9 +307,11 @@ def _qubit_gates(gates, n):
 
 def _native_circuit(pv, gates):
     """_qubit_gates' arrays where the library plans the circuit: a
-    PauliVectorHIP of 2 to 16 qubits in full bases; else None."""
-    from .pauli_vectors import PauliVectorHIP
-    if not isinstance(pv, PauliVectorHIP) or type(pv).apply_ptm is not PauliVectorHIP.apply_ptm:
+    PauliVectorHIP of 2 to 16 qubits in full bases whose apply_ptm nobody
+    replaced; else None."""
+    from .pauli_vectors import hip
+    if not isinstance(pv, hip.PauliVectorHIP) or \
+            getattr(pv.apply_ptm, '__func__', None) is not hip._apply_ptm:
         return None
     n = pv.n_qubits
     if not 2 <= n <= 16 or pv.data_shape != (4,) * n or pv.dim_pauli != (4,) * n:

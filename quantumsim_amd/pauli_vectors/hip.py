@@ -623,3 +623,6 @@ class PauliVectorHIP(PauliVectorBase):
                              dtype=self._dtype, device=self._device)
         self._used_here(self._store)
         return new
+
+
+_apply_ptm = PauliVectorHIP.apply_ptm       # to tell whether a caller replaced it

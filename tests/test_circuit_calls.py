@@ -159,3 +159,36 @@ def test_circuit_without_gates_copies():
     plan.run(x.data_ptr(), y.data_ptr(), None, torch.cuda.current_stream().cuda_stream or None)
     torch.cuda.synchronize()
     assert torch.equal(x, y)
+
+
+def _host_vector(n):
+    """A float64 vector of n qubits without its device memory."""
+    import torch
+    from quantumsim_amd import bases
+    from quantumsim_amd.pauli_vectors import PauliVectorHIP
+    pv = PauliVectorHIP.__new__(PauliVectorHIP)
+    pv.bases = [bases.general(2)] * n
+    pv._shape, pv._dtype = (4,) * n, torch.float64
+    return pv
+
+
+@pytest.mark.parametrize('where', ['class', 'subclass', 'instance'])
+def test_replaced_apply_ptm_sees_every_block(monkeypatch, where):
+    """apply_circuit goes by the vector's apply_ptm wherever that is not the
+    library's own."""
+    from quantumsim_amd.pauli_vectors import PauliVectorHIP
+    rng = np.random.default_rng(5)
+    gates = [(rng.standard_normal((4,) * 4), (q, q + 1)) for q in (0, 2, 1)]
+    assert fusion._native_circuit(_host_vector(4), gates) is not None
+    seen = []
+    pv = _host_vector(4)
+    if where == 'class':
+        monkeypatch.setattr(PauliVectorHIP, 'apply_ptm', lambda self, p, *q: seen.append(q))
+    elif where == 'subclass':
+        pv.__class__ = type('Sub', (PauliVectorHIP,),
+                            {'apply_ptm': lambda self, p, *q: seen.append(q)})
+    else:
+        pv.apply_ptm = lambda p, *q: seen.append(q)
+    monkeypatch.setattr(PauliVectorHIP, 'run_passes', lambda self, *a: True)
+    count = fusion.apply_circuit(pv, gates, 3)
+    assert count == len(seen) and seen == [f.qudits for f in fuse(gates, [4] * 4, 3)]
