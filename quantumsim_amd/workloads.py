@@ -393,7 +393,7 @@ class TrainableCircuit:
         and for the circuits it does not take (windows.LayerBlockPlan)."""
         from .autograd import Gate, cz_ptm
         from .windows import layer_blocks
-        if getattr(self.gates, '__func__', None) is not TrainableCircuit.gates:
+        if getattr(self.gates, '__func__', None) is not _circuit_gates:
             return None
         if ang.dim() != 4 or ang.shape[2:] != (self.n, 2) or \
                 not t1.shape == t2.shape == (ang.shape[0], self.n):
@@ -428,6 +428,9 @@ class TrainableCircuit:
         import torch
         t = target.clamp_min(eps)
         return (target * (torch.log(t) - torch.log(p.clamp_min(eps)))).sum(-1)
+
+
+_circuit_gates = TrainableCircuit.gates      # to tell whether a caller replaced it
 
 
 def random_circuit_batch(n_circuits, seed, n_range=(4, 11), layer_range=(20, 80)):

@@ -219,3 +219,12 @@ def test_overridden_gates_are_used(gates_of):
     class Renamed(TrainableCircuit):         # the same gates: either route
         pass
     _same_gates(gates_of(Renamed(n=4, layers=7), *p), plain)
+
+
+def test_gates_replaced_on_the_class_are_used(gates_of, monkeypatch):
+    tc = TrainableCircuit(n=4, layers=7)
+    p = _params(tc, 2)
+    plain = tc.gates(*p, 3)
+    monkeypatch.setattr(TrainableCircuit, 'gates',
+                        lambda self, ang, t1, t2, fuse_qudits=0: plain[:2])
+    _same_gates(gates_of(tc, *p), plain[:2])
